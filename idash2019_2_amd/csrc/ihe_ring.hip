@@ -19,6 +19,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "ihe_internal.h"
 
@@ -180,293 +181,319 @@ __device__ __forceinline__ int32_t noise_sample_lut(uint64_t u, const uint64_t *
 // v_mfma_i32_32x32x32_i8 per byte plane and K-block of 32 coefficients, four
 // int32 accumulators recombined with shifts mod 2^32 (|partial| <= 2^17).
 //
-// Work items are 32 ciphertexts x 256 samples; a workgroup of 4 waves owns one
-// item at a time, each wave two 32-sample column tiles (so each A operand read
-// feeds eight MFMAs). The workgroups are persistent: each builds the key's B
-// operands once, then takes items from its XCD's counter, so the sample groups
-// of one ciphertext group run side by side on one XCD (sharing its L2).
-//  - B: T's rows 32 ks + 16 h + jj, column j, are the 16 consecutive bytes
-//    u[N - j + 32 ks + 16 h ...] of u[N + x] = S[-x]. LDS holds 16 copies of u
-//    shifted by 0..15 bytes, so every B operand is one aligned 16-byte read;
-//    copies are 2064 bytes apart, which puts neighbouring lanes on different
-//    banks.
-//  - A: per stage of 128 coefficients the workgroup loads the 32 x 128 a-words
-//    (each load instruction reads 8 rows x 128 bytes, one stage ahead of use),
-//    writes their byte planes to LDS (double-buffered, one barrier per stage),
-//    and every wave reads its A operands back lane-linear.
-// Decryption (words j < NS) ends with phase = b - a*s as a float; encryption
-// (all N words; k_encrypt_ae has written a and b = e + messages) adds a*s to
-// b in place. An item's results are written in the next item's first stage.
-constexpr uint32_t kDecCols = 256;              // samples per work item
-constexpr uint32_t kDecUStride = 2 * kN + 16;   // bytes between shifted copies of u
-
-struct DecryptParams {
+// Work items are 32 ciphertexts x 8 TPW column tiles of 32 words (TPW = 1 .. 4
+// tiles a wave; all 1,024 words at TPW = 4). One workgroup of 8 waves per CU
+// holds an item's a-words as byte planes in LDS (128 KB) and stays for further
+// items, taken from its XCD's counter.
+//  - Planes outermost: a wave multiplies all 32 K-blocks of the highest plane
+//    into its tiles' accumulators, shifts them by 8 and goes on with the next
+//    plane (Horner mod 2^32; the MFMA's int32 sums wrap). So a tile costs 16
+//    accumulator registers instead of 64, a wave owns four tiles, and an A
+//    operand read feeds TPW MFMAs. The b words enter with the last shift.
+//  - The B operand of word tile nt and K-block ks depends on nt - ks only: a
+//    wave with adjacent tiles keeps them in a register window that moves by one
+//    block per K-block, one LDS read for TPW MFMAs. Lane (h, c) reads the 16
+//    bytes of u[N + x] = S[-x] from N - 32 (nt - ks) - c + 16 h on; LDS holds
+//    every such 16-byte run (32 KB), consecutive lanes on consecutive runs,
+//    which leaves no bank conflicts (shifted copies of u conflict once per 16
+//    lanes wherever they lie).
+//  - A: each thread loads 16 pieces of four words (16 lanes x 16 bytes of a
+//    row), recodes them to digits and writes each plane's four bytes. The rows
+//    of the planes' 16-byte cells are XORed with the K half and the K-block's
+//    parity, which spreads the writes over the banks.
+//  - Everything that touches memory is spread over the K-block steps of some
+//    pass: results of the item before in plane 3's pass, b words in plane 2's,
+//    the next item's a-words in plane 1's and 0's (from plane 3's on where the
+//    registers allow, TPW < 4), their recoding in plane 0's. A wave that issues
+//    64 loads or stores in a row stalls on the memory pipe and keeps the matrix
+//    pipe idle. Two barriers an item: planes 3 and 2 are rewritten between the
+//    passes 1 and 0, planes 1 and 0 in the next item's pass 3.
+// Decryption (words j < NS) ends with phase = b - a*s as a float (u negated);
+// encryption (all N words; k_encrypt_ae has written a and b = e + messages)
+// adds a*s to b in place.
+//
+// What bounds it: at 242,646 ciphertexts x 1,024 words 0.75 ms (0.92 ms with 64
+// accumulators a tile, two tiles a wave and 256-word items). The matrix pipe is
+// busy 82 % of the cycles (58 % before), and the chip then lowers its clock to
+// 1.7 GHz for power; with the MFMAs left out the same kernel takes 0.52 ms
+// (5.7 TB/s). At 45,011 x 203 words: 0.064 ms (0.083 ms before), HBM and the last,
+// half-filled round of workgroups.
+struct RingParams {
   const int32_t *in;
   float *out;     // decryption: phases [num_cts][ns]
   int32_t *bout;  // encryption: the ciphertexts of `in` (same buffer), b halves updated
   uint32_t num_cts, ns, col_groups, num_items;
-  // kRingQueueWords zero words: items are taken from per-XCD counters; null:
-  // workgroup x takes items x, x + 8 ... of its XCD's range
+  // kRingQueueWords zero words: a workgroup's first item is fixed, the others
+  // are taken from its XCD's counter; null: every gridDim / 8-th of its range
   uint32_t *queue;
 };
 
 
 // u[y] = S[N - y]: s[N - y] for 1 <= y <= N, -s[2N - y] for N < y < 2N, else 0
-// (key words in LDS).
+// (key words in LDS); NEG: its negative.
+template <bool NEG>
 __device__ __forceinline__ uint32_t u_byte(uint32_t y, const uint32_t *kw) {
-  if (y >= 1 && y <= kN) {
-    const uint32_t m = kN - y;
-    return (kw[m / 32] >> (m % 32)) & 1u;
-  }
-  if (y > kN && y < 2 * kN) {
-    const uint32_t m = 2 * kN - y;
-    return ((kw[m / 32] >> (m % 32)) & 1u) ? 0xFFu : 0u;
-  }
-  return 0u;
+  const uint32_t m = (0u - y) & (kN - 1);
+  const uint32_t bit = y ? (kw[m / 32] >> (m % 32)) & 1u : 0u;
+  return bit * ((y > kN) != NEG ? 0xFFu : 1u);
 }
 
-// TW column tiles per wave, 8 / TW waves per workgroup: TW = 2 reads each A
-// operand into 8 MFMAs at 2 waves per SIMD, TW = 1 into 4 at 4 waves per SIMD.
-template <bool ENC, int TW>
-__global__ __launch_bounds__(64 * (8 / TW)) __attribute__((amdgpu_waves_per_eu(4 / TW, 4 / TW)))
-void k_ring_mfma(DecryptParams P, KeyBits key) {
+constexpr uint32_t kRuns = 2 * kN - 16;  // 16-byte runs of u that B operands are made of
+constexpr uint32_t kRingThreads = 512, kRingWaves = kRingThreads / 64;
+
+struct RingLds {
+  uint32_t planes[4][kN / 32][256];  // [plane][K-block][k half][row, swizzled][4 dwords]
+  uint32_t u[kRuns][4];  // run e: bytes u[e + 1 .. e + 16]
+  uint32_t next;                 // the item after the next one
+};
+static_assert(sizeof(RingLds) <= 160 * 1024, "one workgroup's LDS");
+
+template <bool ENC, int TPW>
+__global__ __launch_bounds__(kRingThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void k_ring_mfma(RingParams P, KeyBits key) {
   typedef int int4v __attribute__((ext_vector_type(4)));
   typedef int int16v __attribute__((ext_vector_type(16)));
-  constexpr uint32_t kDecWaves = 8 / TW;
-  // loader role: kLpr lanes per ciphertext row, each loading kNl 16-byte
-  // pieces kStride words apart per stage (each load instruction reads whole
-  // 128-byte lines of 64 * 16 / (16 * kLpr) rows)
-  constexpr uint32_t kLpr = 2 * kDecWaves, kNl = 32 / kLpr, kStride = 4 * kLpr;
-  __shared__ __attribute__((aligned(16))) uint8_t U[16 * kDecUStride];
-  // byte planes of one stage: [buffer][kb][plane][k half][row][4 dwords]
-  __shared__ __attribute__((aligned(16))) uint32_t planes[2][4][4][2][32][4];
+  typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+  constexpr int kRsrc3 = 0x00020000;  // raw buffer descriptor, dword 3
+  constexpr uint32_t kDrop = 0x80000000u;  // an offset past every buffer: loads 0, stores nothing
+  constexpr uint32_t kCtBytes = kCtWords * 4;
+  constexpr bool kEarly = TPW < 4;  // registers left to load the next item from pass 3 on
+  __shared__ __attribute__((aligned(16))) RingLds S;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const uint32_t h = lane / 32, c = lane % 32;
-  __shared__ uint32_t kw[kN / 32];
-  if (threadIdx.x < kN / 32) kw[threadIdx.x] = key.w[threadIdx.x];
-  __syncthreads();
-  // U[s * kDecUStride + y] = u[y + s]
-  for (uint32_t t = threadIdx.x; t < 16 * (2 * kN / 4); t += 64 * kDecWaves) {
-    const uint32_t sh = t / (2 * kN / 4), d = t % (2 * kN / 4);
-    uint32_t v = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) v |= u_byte(4 * d + sh + i, kw) << (8 * i);
-    *(uint32_t *)(U + sh * kDecUStride + 4 * d) = v;
-  }
-  __syncthreads();
-  // items of XCD x (blocks x, x + 8, ...): a contiguous range, walked in order.
-  // From the counter, a workgroup takes the next item when it starts one, so
-  // the sample groups of a ciphertext group run side by side all the way
-  // (a fixed stride lets workgroups drift apart, and their shared a-words
-  // then leave L2 between the reads).
-  const uint32_t xcd = blockIdx.x % 8, per_xcd = gridDim.x / 8, slot = blockIdx.x / 8;
+  const uint32_t lim = ENC ? kN : P.ns;
+  const uint32_t xcd = blockIdx.x % 8, per_xcd = gridDim.x / 8;
   const uint32_t chunk = (P.num_items + 7) / 8;
   const uint32_t it_beg = min(xcd * chunk, P.num_items);
   const uint32_t it_end = min((xcd + 1) * chunk, P.num_items);
-  // the item after the k-th is announced in s_next[(k + 1) % 2]
-  __shared__ uint32_t s_next[2];
-  const uint32_t r = threadIdx.x / kLpr, cq = threadIdx.x % kLpr;
-  // an item's ciphertext group starts at a wave-uniform address; a loader
-  // thread adds its row (clamped to the last ciphertext) as a byte offset
-  auto group_of = [&](uint32_t item) {
-    return (const char *)(P.in + (size_t)(item / P.col_groups) * 32 * kCtWords);
+  // this item, the next (loaded meanwhile) and, in S.next, the one after it
+  uint32_t item = it_beg + blockIdx.x / 8, next = item + per_xcd;
+
+  // loader role: words 64 i + 4 lc .. + 3 of row lr, i < 16
+  const uint32_t lr = threadIdx.x / 16, lc = threadIdx.x % 16;
+  const uint32_t wpar = lc / 8, whalf = (lc % 8) / 4;
+  uint32_t *const wp =
+      &S.planes[0][wpar][whalf * 128 + ((lr ^ (4 * whalf) ^ (2 * wpar)) * 4) + lc % 4];
+  u32x4v q[16];
+  auto rows_of = [&](uint32_t it) { return min(32u, P.num_cts - (it / P.col_groups) * 32); };
+  auto in_rsrc = [&](uint32_t it, bool on) {
+    return __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(P.in + (size_t)(it / P.col_groups) * 32 * kCtWords), (short)0,
+        on ? (int)(32 * kCtBytes) : 0, kRsrc3);
   };
-  auto row_off = [&](uint32_t item) {
-    return (min(r, P.num_cts - 1 - (item / P.col_groups) * 32) * kCtWords + 4 * cq) * 4;
+  auto a_off = [&](uint32_t it) { return min(lr, rows_of(it) - 1) * kCtBytes + lc * 16; };
+  auto load_a = [&](const __amdgpu_buffer_rsrc_t &R, uint32_t vo, int i) {
+    q[i] = __builtin_bit_cast(u32x4v, __builtin_amdgcn_raw_buffer_load_b128(R, vo + 256 * i, 0, 0));
   };
-  int4v xr[kNl];
-  uint32_t item = it_beg + slot;
-  if (P.queue) {
-    if (threadIdx.x == 0) s_next[0] = it_beg + atomicAdd(&P.queue[xcd], 1u);
-    __syncthreads();
-    item = __builtin_amdgcn_readfirstlane(s_next[0]);
-  }
-  if (item < it_end) {
-    const char *g = group_of(item);
-    const uint32_t o = row_off(item);
+  auto put = [&](int p, int i) { wp[p * 8192 + i * 512] = q[i][p]; };
+  // piece i: four words -> their digits by plane; planes 3 and 2 written
+  auto recode = [&](int i) {
+    u32x4v y;
 #pragma unroll
-    for (uint32_t i = 0; i < kNl; ++i) xr[i] = *(const int4v *)(g + o + 4 * kStride * i);
-  }
-  uint32_t next = 0;
-  // An item's results are written in the next item's first stage, after that
-  // stage's loads are issued: the memory counter covers stores too, so waits
-  // for loads issued after the stores would also wait for the stores.
-  int16v acc[TW][4];
-  uint32_t bw[16];  // first column tile's b words, loaded in the last stage
-  bool pend = false;
-  uint32_t p_ct0 = 0, p_jw = 0;
-  // decryption needs the words j < NS, encryption all N
-  const uint32_t lim = ENC ? kN : P.ns;
-  auto whole = [&](uint32_t ct0, uint32_t jw) {
-    return ct0 + 32 <= P.num_cts && jw + 32 * TW <= lim;
+    for (int k = 0; k < 4; ++k) y[k] = (q[i][k] + 0x80808080u) ^ 0x80808080u;
+    const uint32_t t0 = __builtin_amdgcn_perm(y[1], y[0], 0x05010400u);
+    const uint32_t t1 = __builtin_amdgcn_perm(y[1], y[0], 0x07030602u);
+    const uint32_t t2 = __builtin_amdgcn_perm(y[3], y[2], 0x05010400u);
+    const uint32_t t3 = __builtin_amdgcn_perm(y[3], y[2], 0x07030602u);
+    q[i][0] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
+    q[i][1] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
+    q[i][2] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
+    q[i][3] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
+    put(3, i);
+    put(2, i);
   };
-  // whole tiles: one wave-uniform base per item, 32-bit byte offsets (row v of
-  // a tile is ciphertext ct0 + 8 (v / 4) + 4 h + v % 4)
-  auto in_off = [&](uint32_t jw, int v) {
-    return (4 * h * kCtWords + kN + jw + c + (8 * (v / 4) + (v % 4)) * kCtWords) * 4;
-  };
-  auto load_bw1 = [&](uint32_t ct0, uint32_t jw, uint32_t (&bw1)[16]) {
-    const char *in_base = (const char *)(P.in + (size_t)ct0 * kCtWords);
+
+  {
+    const __amdgpu_buffer_rsrc_t R = in_rsrc(item < it_end ? item : 0, item < it_end);
+    const uint32_t vo = a_off(item < it_end ? item : 0);
 #pragma unroll
-    for (int v = 0; v < 16; ++v) bw1[v] = *(const uint32_t *)(in_base + in_off(jw, v) + 128);
+    for (int i = 0; i < 16; ++i) load_a(R, vo, i);
+  }
+  uint32_t taken = 0;
+  if (P.queue && threadIdx.x == 0) taken = atomicAdd(&P.queue[xcd], 1u);
+  // u itself, in the space of the planes, then its runs
+  uint32_t *const kw = &S.planes[0][0][0], *const u0 = &S.planes[1][0][0];
+  if (threadIdx.x < kN / 32) kw[threadIdx.x] = key.w[threadIdx.x];
+  __syncthreads();
+  {
+    uint32_t v = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) v |= u_byte<!ENC>(4 * threadIdx.x + i, kw) << (8 * i);
+    u0[threadIdx.x] = v;
+  }
+  if (P.queue && threadIdx.x == 0) S.next = it_beg + per_xcd + taken;
+  __syncthreads();
+  if (threadIdx.x < kRuns / 4) {  // runs 4 t .. 4 t + 3: dwords t .. t + 4 of u
+    uint32_t x[5];
+#pragma unroll
+    for (uint32_t i = 0; i < 5; ++i) x[i] = u0[threadIdx.x + i];
+#pragma unroll
+    for (int s = 1; s <= 4; ++s) {
+      u32x4v v;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = s < 4 ? __builtin_amdgcn_alignbyte(x[k + 1], x[k], s) : x[k + 1];
+      *(u32x4v *)S.u[4 * threadIdx.x + s - 1] = v;
+    }
+  }
+  if (P.queue) next = __builtin_amdgcn_readfirstlane(S.next);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) recode(i);
+  __syncthreads();
+
+  // A operand addresses of this lane in even and odd K-blocks
+  const uint8_t *const ra0 = (const uint8_t *)&S.planes[0][0][h * 128 + ((c ^ (4 * h)) * 4)];
+  const uint8_t *const ra1 = (const uint8_t *)&S.planes[0][0][h * 128 + ((c ^ (4 * h) ^ 2) * 4)];
+  const uint32_t ostride = ENC ? kCtBytes : P.ns * 4;
+  int16v br[TPW];  // an item's b words, then its results
+  uint32_t vo[TPW];
+  uint32_t p_item = 0, p_rows = 0;  // the item of the results in br; 0 rows: none
+  auto out_rsrc = [&](uint32_t it, bool on) {
+    const size_t ct0 = (size_t)(it / P.col_groups) * 32;
+    return __builtin_amdgcn_make_buffer_rsrc(
+        ENC ? (void *)(P.bout + ct0 * kCtWords) : (void *)(P.out + ct0 * P.ns), (short)0,
+        on ? (int)(32 * ostride) : 0, kRsrc3);
   };
-  // decryption: phase = b - a*s; encryption: b += a*s in place
-  auto finish = [&](uint32_t ct0, uint32_t jw, const uint32_t (&bw1)[16]) {
-    auto as_of = [&](int t, int v) {
-      return ((((((uint32_t)acc[t][3][v] << 8) + (uint32_t)acc[t][2][v]) << 8) +
-               (uint32_t)acc[t][1][v]) << 8) + (uint32_t)acc[t][0][v];
+  // a value that what depends on it is computed from where it is used, not earlier
+  auto late = [](uint32_t x) {
+    asm volatile("" : "+v"(x));
+    return x;
+  };
+  // value v of a tile: row m + 4 h of the item, m = 8 (v / 4) + v % 4
+  auto row_of = [](int v) -> uint32_t { return 8 * (v / 4) + v % 4; };
+  auto store = [&](const __amdgpu_buffer_rsrc_t &R, int i) {
+    const int v = i / TPW, t = i % TPW;
+    __builtin_amdgcn_raw_buffer_store_b32(br[t][v], R, vo[t], row_of(v) * ostride, 2);
+  };
+  auto store_part = [&]() {
+    const __amdgpu_buffer_rsrc_t R = out_rsrc(p_item, true);
+    const uint32_t r0 = late(4 * h);
+#pragma unroll
+    for (int i = 0; i < 16 * TPW; ++i) {
+      const int v = i / TPW, t = i % TPW;
+      __builtin_amdgcn_raw_buffer_store_b32(
+          br[t][v], R, row_of(v) + r0 < p_rows ? vo[t] : kDrop, row_of(v) * ostride, 2);
+    }
+  };
+#pragma unroll
+  for (int t = 0; t < TPW; ++t) br[t] = int16v{}, vo[t] = kDrop;
+
+  while (item < it_end) {
+    const uint32_t rows = rows_of(item);
+    const uint32_t nt0 = (item % P.col_groups) * (kRingWaves * TPW) + wave * TPW;
+    const bool active = nt0 * 32 < lim, full = rows == 32, more = next < it_end;
+    const __amdgpu_buffer_rsrc_t nr = in_rsrc(more ? next : item, more);
+    const uint32_t nvo = a_off(more ? next : item);
+    const int4v *const bl = (const int4v *)S.u + (kN - 1 - 32 * nt0 - c + 16 * h);
+    int16v acc[TPW];
+    // plane p's K-blocks; hook(ks) issues the step's share of other work, and a
+    // scheduling barrier keeps it there
+    auto pass = [&](int p, auto hook) {
+      constexpr int kSlots = TPW + 2;  // the block of tile t at K-block ks: slot (t - ks) mod kSlots
+      auto slot = [](int d) { return (d + 32 * kSlots) % kSlots; };
+      int4v w[kSlots], a[3];
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) w[t] = bl[-32 * t];
+      w[slot(-1)] = bl[32];
+      a[0] = *(const int4v *)(ra0 + p * 32768);
+      a[1] = *(const int4v *)(ra1 + p * 32768 + 1024);
+      if (p < 3) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) acc[t] = p == 0 ? (acc[t] << 8) + br[t] : acc[t] << 8;
+      }
+#pragma unroll
+      for (int ks = 0; ks < 32; ++ks) {
+        if (ks + 2 < 32) {
+          w[slot(-(ks + 2))] = bl[32 * (ks + 2)];
+          a[(ks + 2) % 3] = *(const int4v *)((ks & 1 ? ra1 : ra0) + p * 32768 + (ks + 2) * 1024);
+        }
+        hook(ks);
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+          acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+              a[ks % 3], w[slot(t - ks)], p == 3 && ks == 0 ? int16v{} : acc[t], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     };
-    if (whole(ct0, jw)) {  // streaming (nt) stores: outputs are not re-read here
-      char *out_base = ENC ? (char *)(P.bout + (size_t)ct0 * kCtWords)
-                           : (char *)(P.out + (size_t)ct0 * P.ns);
-      const uint32_t out_lane = (4 * h * P.ns + jw + c) * 4;
+    if (P.queue && threadIdx.x == 0) taken = atomicAdd(&P.queue[xcd], 1u);
+    // whole results go out in pass 3, a partial group's (or an idle wave's) at once
+    const bool whole = active && p_rows == 32;
+    if (!whole && p_rows) store_part();
+    const __amdgpu_buffer_rsrc_t orr = out_rsrc(p_item, whole);
+    const __amdgpu_buffer_rsrc_t ir = in_rsrc(item, full);
+    uint32_t vb[TPW];
+    if (active) {
+      pass(3, [&](int ks) {
+        if (ks < 16) {
+          put(1, ks);
+          put(0, ks);
+          if constexpr (kEarly) load_a(nr, nvo, ks);
+        }
 #pragma unroll
-      for (int t = 0; t < TW; ++t) {
+        for (int i = ks * TPW / 2; i < (ks + 1) * TPW / 2; ++i) store(orr, i);
+      });
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const uint32_t as = as_of(t, v), b = t == 0 ? bw[v] : bw1[v];
-          if constexpr (ENC)
-            __builtin_nontemporal_store((int32_t)(b + as),
-                                        (int32_t *)(out_base + in_off(jw, v) + 128 * t));
-          else
-            __builtin_nontemporal_store(
-                (float)(int32_t)(b - as) * 0x1p-32f,
-                (float *)(out_base + out_lane + (8 * (v / 4) + (v % 4)) * P.ns * 4 + 128 * t));
+      for (int t = 0; t < TPW; ++t) {
+        const uint32_t j = (nt0 + t) * 32 + c;
+        vb[t] = j < lim ? 4 * h * kCtBytes + (kN + j) * 4 : kDrop;
+        vo[t] = j < lim ? 4 * h * ostride + ((ENC ? kN : 0) + j) * 4 : kDrop;
+      }
+      pass(2, [&](int ks) {
+#pragma unroll
+        for (int i = ks * TPW / 2; i < (ks + 1) * TPW / 2; ++i) {
+          const int v = i / TPW, t = i % TPW;
+          br[t][v] = __builtin_amdgcn_raw_buffer_load_b32(ir, vb[t], row_of(v) * kCtBytes, 0);
+        }
+      });
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        put(1, i);
+        put(0, i);
+        if constexpr (kEarly) load_a(nr, nvo, i);
+      }
+    }
+    __syncthreads();
+    if (P.queue && threadIdx.x == 0) S.next = it_beg + per_xcd + taken;
+    if (active) {
+      pass(1, [&](int ks) {
+        if (!kEarly && ks >= 16 && ks % 2 == 0) load_a(nr, nvo, (ks - 16) / 2);
+      });
+      if (!full) {
+        const __amdgpu_buffer_rsrc_t pr = in_rsrc(item, true);
+        const uint32_t r0 = late(4 * h);
+#pragma unroll
+        for (int i = 0; i < 16 * TPW; ++i) {
+          const int v = i / TPW, t = i % TPW;
+          br[t][v] = __builtin_amdgcn_raw_buffer_load_b32(
+              pr, row_of(v) + r0 < rows ? vb[t] : kDrop, row_of(v) * kCtBytes, 0);
         }
       }
-      return;
-    }
-    const char *ag = (const char *)(P.in + (size_t)ct0 * kCtWords);
-    const uint32_t jc1 = min(jw + 32 + c, lim - 1);
+      pass(0, [&](int ks) {
+        if (!kEarly && ks < 16 && ks % 2 == 0) load_a(nr, nvo, 8 + ks / 2);
+        if (ks >= 16) recode(ks - 16);
+      });
 #pragma unroll
-    for (int t = 0; t < TW; ++t) {
-      const uint32_t j = jw + 32 * t + c;
-      if (jw + 32 * t >= lim) continue;
-      if (t == 1) {
+      for (int t = 0; t < TPW; ++t)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const uint32_t ct = min(ct0 + 8 * (v / 4) + 4 * h + (v % 4), P.num_cts - 1);
-          bw[v] = *(const uint32_t *)(ag + ((ct - ct0) * kCtWords + kN + jc1) * 4);
-        }
+        for (int v = 0; v < 16; ++v)
+          br[t][v] = ENC ? acc[t][v] : __builtin_bit_cast(int, (float)acc[t][v] * 0x1p-32f);
+    } else {
+      if constexpr (!kEarly) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) load_a(nr, nvo, i);
       }
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const uint32_t ct = ct0 + 8 * (v / 4) + 4 * h + (v % 4);
-        const uint32_t as = as_of(t, v);
-        if (ct >= P.num_cts || j >= lim) continue;
-        if constexpr (ENC)
-          P.bout[(size_t)ct * kCtWords + kN + j] = (int32_t)(bw[v] + as);
-        else
-          P.out[(size_t)ct * P.ns + j] = (float)(int32_t)(bw[v] - as) * 0x1p-32f;
-      }
+      for (int i = 0; i < 16; ++i) recode(i);
     }
-  };
-  // byte planes of the loaded stage into planes[buf]
-  auto recode = [&](uint32_t buf) {
-#pragma unroll
-    for (uint32_t i = 0; i < kNl; ++i) {
-      // coefficients w .. w + 3 of the stage: K-block w / 32, bytes k0 .. k0 + 3
-      const uint32_t w = kStride * i + 4 * cq, kb = w / 32, k0 = w % 32;
-      uint32_t y[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) y[q] = ((uint32_t)xr[i][q] + 0x80808080u) ^ 0x80808080u;
-      const uint32_t t0 = __builtin_amdgcn_perm(y[1], y[0], 0x05010400u);
-      const uint32_t t1 = __builtin_amdgcn_perm(y[1], y[0], 0x07030602u);
-      const uint32_t t2 = __builtin_amdgcn_perm(y[3], y[2], 0x05010400u);
-      const uint32_t t3 = __builtin_amdgcn_perm(y[3], y[2], 0x07030602u);
-      planes[buf][kb][0][k0 / 16][r][(k0 % 16) / 4] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
-      planes[buf][kb][1][k0 / 16][r][(k0 % 16) / 4] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
-      planes[buf][kb][2][k0 / 16][r][(k0 % 16) / 4] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
-      planes[buf][kb][3][k0 / 16][r][(k0 % 16) / 4] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
-    }
-  };
-  // stage st's K-blocks. A wave with any active tile multiplies all of them
-  // (a tile past NS costs only its multiplications: its B reads stay inside
-  // u), so the K-block loop has no branches and one wait per K-block.
-  auto multiply = [&](uint32_t st, uint32_t jw) {
-    const uint32_t buf = st & 1;
-#pragma unroll
-    for (uint32_t kb = 0; kb < 4; ++kb) {
-      const uint32_t ks = 4 * st + kb;
-      int4v a[4], bop[TW];
-#pragma unroll
-      for (int p = 0; p < 4; ++p) a[p] = *(const int4v *)&planes[buf][kb][p][h][c][0];
-#pragma unroll
-      for (int t = 0; t < TW; ++t) {
-        const uint32_t start = kN - (jw + 32 * t) + 32 * ks - c + 16 * h;  // in [1, 2N - 16]
-        const uint32_t sh = start & 15u;
-        bop[t] = *(const int4v *)(U + sh * kDecUStride + (start - sh));
-      }
-#pragma unroll
-      for (int t = 0; t < TW; ++t)
-#pragma unroll
-        for (int p = 0; p < 4; ++p)
-          acc[t][p] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[p], bop[t], acc[t][p], 0, 0, 0);
-    }
-  };
-  for (uint32_t k = 1; item < it_end; item = next, k ^= 1) {
-    const uint32_t ct0 = (item / P.col_groups) * 32;
-    const uint32_t jw = (item % P.col_groups) * kDecCols + wave * 32 * TW;
-    const char *ag = group_of(item);
-    const uint32_t ao = row_off(item);
-    const uint32_t jc0 = min(jw + c, lim - 1);
-    {
-      // first stage: take the next item from the counter (announced at this
-      // stage's barrier), write the previous item's results after issuing
-      // this stage's loads
-      const bool grab = P.queue && threadIdx.x == 0;
-      uint32_t taken = 0;
-      if (grab) taken = atomicAdd(&P.queue[xcd], 1u);  // first used at the barrier
-      recode(0);
-      uint32_t bw1[16];
-      if (TW == 2 && pend && whole(p_ct0, p_jw)) load_bw1(p_ct0, p_jw, bw1);
-#pragma unroll
-      for (uint32_t i = 0; i < kNl; ++i) xr[i] = *(const int4v *)(ag + ao + 4 * (128 + kStride * i));
-      if (pend) finish(p_ct0, p_jw, bw1);
-#pragma unroll
-      for (int t = 0; t < TW; ++t)
-#pragma unroll
-        for (int p = 0; p < 4; ++p) acc[t][p] = int16v{};
-      if (grab) s_next[k] = taken;
-      __syncthreads();
-      if (jw < lim) multiply(0, jw);
-    }
-    for (uint32_t st = 1; st < kN / 128; ++st) {
-      recode(st & 1);
-      if (st + 1 < kN / 128) {
-#pragma unroll
-        for (uint32_t i = 0; i < kNl; ++i)
-          xr[i] = *(const int4v *)(ag + ao + 4 * (128 * (st + 1) + kStride * i));
-      } else {
-        // the first column tile's b words, then the next item's first stage:
-        // both arrive while this stage multiplies
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const uint32_t ct = min(ct0 + 8 * (v / 4) + 4 * h + (v % 4), P.num_cts - 1);
-          bw[v] = *(const uint32_t *)(ag + ((ct - ct0) * kCtWords + kN + jc0) * 4);
-        }
-        next = P.queue ? it_beg + __builtin_amdgcn_readfirstlane(s_next[k]) : item + per_xcd;
-        if (next < it_end) {
-          const char *ng = group_of(next);
-          const uint32_t no = row_off(next);
-#pragma unroll
-          for (uint32_t i = 0; i < kNl; ++i) xr[i] = *(const int4v *)(ng + no + 4 * kStride * i);
-        }
-      }
-      __syncthreads();
-      if (jw < lim) multiply(st, jw);
-    }
-    pend = true;
-    p_ct0 = ct0;
-    p_jw = jw;
+    p_item = item;
+    p_rows = active ? rows : 0;
+    __syncthreads();
+    item = next;
+    next = P.queue ? (uint32_t)__builtin_amdgcn_readfirstlane(S.next) : next + per_xcd;
   }
-  if (pend) {
-    uint32_t bw1[16];
-    if (TW == 2 && whole(p_ct0, p_jw)) load_bw1(p_ct0, p_jw, bw1);
-    finish(p_ct0, p_jw, bw1);
-  }
-  // every workgroup has taken its last (empty) item: the last one to finish
-  // clears the counters for the next launch
+  if (p_rows) store_part();
+  // the last workgroup to finish clears the counters for the next launch
   if (P.queue && threadIdx.x == 0) {
     if (atomicAdd(&P.queue[8], 1u) == gridDim.x - 1)
       for (uint32_t i = 0; i <= 8; ++i) atomicExch(&P.queue[i], 0u);
@@ -608,35 +635,52 @@ __global__ __launch_bounds__(256) void k_encrypt_ae(EncryptParams P) {
 // x column groups of 1024 words) stays far inside the 32-bit counters.
 constexpr uint32_t kNoallocMaxCts = 1u << 26;
 
-// IHE_RING_TILES = 1 or 2 column tiles per wave (default 2); IHE_RING_QUEUE=0
-// gives the workgroups fixed items instead of the counters
+// Column tiles per wave (TPW). A round of workgroups, one per CU, takes about
+// 5 us for an item's a-words and 2.5 us for each tile that a SIMD's waves own
+// (waves w and w + 4 share a SIMD); fewer tiles a wave make more items, which
+// pays where the ciphertexts alone leave CUs idle (33 ciphertexts x 1,024
+// words: 13.4 us at TPW = 1, 24.7 us at 4; 242,646: 1,024 and 742 us), and
+// three or four tiles keep NS = 300 or 512 to one wave per SIMD (242,646 x 300:
+// 372 us at TPW = 3, 384 us at 2). Ties go to more tiles, which read less LDS
+// (45,011 x 512: 82.6 us at 4, 87.4 us at 2). IHE_RING_TILES = 1 .. 4 sets it;
+// IHE_RING_QUEUE=0 gives the workgroups fixed items instead of the counters.
+uint32_t ring_tiles_per_wave(uint32_t groups, uint32_t tiles, uint32_t num_cus) {
+  const char *e = std::getenv("IHE_RING_TILES");
+  if (e && e[0] >= '1' && e[0] <= '4' && !e[1]) return (uint32_t)(e[0] - '0');
+  uint64_t best = ~0ull;
+  uint32_t tpw = 1;
+  for (uint32_t t = 1; t <= 4; ++t) {
+    const uint32_t per_item = kRingWaves * t, cg = (tiles + per_item - 1) / per_item;
+    const uint64_t rounds = ((uint64_t)groups * cg + num_cus - 1) / num_cus;
+    const bool one_wave = cg == 1 && tiles <= kRingWaves / 2 * t;  // per SIMD
+    const uint64_t cost = rounds * (2 + (one_wave ? t : 2 * t));
+    if (cost <= best) {
+      best = cost;
+      tpw = t;
+    }
+  }
+  return tpw;
+}
+
+// Launch shape: one persistent workgroup per CU, a multiple of the 8 XCDs.
 template <bool ENC>
-void launch_ring_on(hipStream_t stream, DecryptParams P, const KeyBits &key, uint32_t blocks,
-                    uint32_t *queue) {
+void launch_ring(hipStream_t stream, RingParams P, const KeyBits &key, uint32_t num_cus,
+                 uint32_t *queue) {
   static_assert(kRingQueueWords >= 9, "eight XCD counters and a finished count");
   const char *q = std::getenv("IHE_RING_QUEUE");
   P.queue = (q && std::strcmp(q, "0") == 0) ? nullptr : queue;
-  const char *e = std::getenv("IHE_RING_TILES");
-  if (e && std::strcmp(e, "1") == 0)
-    hipLaunchKernelGGL((k_ring_mfma<ENC, 1>), dim3(blocks), dim3(64 * 8), 0, stream, P, key);
-  else
-    hipLaunchKernelGGL((k_ring_mfma<ENC, 2>), dim3(blocks), dim3(64 * 4), 0, stream, P, key);
-}
-
-template <bool ENC>
-void launch_ring(ihe_ctx *ctx, DecryptParams P, const KeyBits &key, uint32_t blocks) {
-  launch_ring_on<ENC>(ctx->stream, P, key, blocks, ctx->d_ring_queue);
-}
-
-// Decrypt launch shape: items of 32 ciphertexts x 32 * kDecCols words, run by
-// persistent workgroups, two per CU, a multiple of the 8 XCDs.
-DecryptParams decrypt_params(const int32_t *d_in, uint32_t num_samples, uint32_t num_cts,
-                             float *d_out, uint32_t num_cus, uint32_t &blocks) {
-  const uint32_t col_groups = (num_samples + kDecCols - 1) / kDecCols;
-  DecryptParams P{d_in, d_out, nullptr, num_cts, num_samples, col_groups,
-                  ((num_cts + 31) / 32) * col_groups, nullptr};
-  blocks = std::min<uint32_t>((num_cus * 2 + 7) / 8 * 8, (P.num_items + 7) / 8 * 8);
-  return P;
+  const uint32_t tiles = ((ENC ? kN : P.ns) + 31) / 32, groups = (P.num_cts + 31) / 32;
+  const uint32_t tpw = ring_tiles_per_wave(groups, tiles, num_cus);
+  P.col_groups = (tiles + kRingWaves * tpw - 1) / (kRingWaves * tpw);
+  P.num_items = groups * P.col_groups;
+  const dim3 grid(std::min<uint32_t>((num_cus + 7) / 8 * 8, (P.num_items + 7) / 8 * 8));
+  const dim3 block(kRingThreads);
+  switch (tpw) {
+    case 1: hipLaunchKernelGGL((k_ring_mfma<ENC, 1>), grid, block, 0, stream, P, key); break;
+    case 2: hipLaunchKernelGGL((k_ring_mfma<ENC, 2>), grid, block, 0, stream, P, key); break;
+    case 3: hipLaunchKernelGGL((k_ring_mfma<ENC, 3>), grid, block, 0, stream, P, key); break;
+    default: hipLaunchKernelGGL((k_ring_mfma<ENC, 4>), grid, block, 0, stream, P, key); break;
+  }
 }
 
 __global__ void k_clear_words(uint32_t *p, uint32_t n) {
@@ -738,16 +782,12 @@ int ihe_encrypt(ihe_ctx *ctx, const ihe_key *key, const ihe_layout *layout, uint
   const char *force = std::getenv("IHE_ENCRYPT_KERNEL");
   if (!(force && std::strcmp(force, "valu") == 0)) {
     // a and b = e + messages, then b += a*s on the MFMA kernel
-    const uint32_t col_groups = kN / kDecCols;
-    DecryptParams D{d_out, nullptr, d_out, P.num_cts, NS, col_groups,
-                    ((P.num_cts + 31) / 32) * col_groups, nullptr};
-    const uint32_t blocks = std::min<uint32_t>(((uint32_t)ctx->num_cus * 2 + 7) / 8 * 8,
-                                               (D.num_items + 7) / 8 * 8);
+    const RingParams D{d_out, nullptr, d_out, P.num_cts, NS, 0, 0, nullptr};
     ScopedTimer t(ctx, IHE_TIMER_ENCRYPT);
     static_assert(kN / 4 == 256, "a thread per four words of a ciphertext");
     hipLaunchKernelGGL(k_encrypt_ae, dim3(std::min<uint32_t>(P.num_cts, (uint32_t)ctx->num_cus * 8)),
                        dim3(256), 0, ctx->stream, P);
-    launch_ring<true>(ctx, D, key->bits, blocks);
+    launch_ring<true>(ctx->stream, D, key->bits, (uint32_t)ctx->num_cus, ctx->d_ring_queue);
     IHE_HIP(hipGetLastError());
     return IHE_OK;
   }
@@ -772,10 +812,8 @@ int ihe_decrypt(ihe_ctx *ctx, const ihe_key *key, uint32_t num_samples, const in
   ScopedTimer t(ctx, IHE_TIMER_DECRYPT);
   const char *force = std::getenv("IHE_DECRYPT_KERNEL");
   if (!(force && std::strcmp(force, "valu") == 0)) {
-    uint32_t blocks;
-    const DecryptParams P =
-        decrypt_params(d_in, num_samples, num_cts, d_out, (uint32_t)ctx->num_cus, blocks);
-    launch_ring<false>(ctx, P, key->bits, blocks);
+    const RingParams P{d_in, d_out, nullptr, num_cts, num_samples, 0, 0, nullptr};
+    launch_ring<false>(ctx->stream, P, key->bits, (uint32_t)ctx->num_cus, ctx->d_ring_queue);
     IHE_HIP(hipGetLastError());
     return IHE_OK;
   }
@@ -810,11 +848,10 @@ int ihe_decrypt_noalloc(const int32_t *key, uint32_t num_samples, const int32_t 
   NoallocDevice D;
   if (int rc = noalloc_device(dev, D)) return rc;
   hipStream_t stream = static_cast<hipStream_t>(hip_stream);
-  uint32_t blocks;
-  const DecryptParams P = decrypt_params(d_in, num_samples, num_cts, d_out, D.num_cus, blocks);
+  const RingParams P{d_in, d_out, nullptr, num_cts, num_samples, 0, 0, nullptr};
   // the counters start at zero (a fill kernel: no memset node under capture)
   hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(64), 0, stream, D.scratch, kRingQueueWords);
-  launch_ring_on<false>(stream, P, bits, blocks, D.scratch);
+  launch_ring<false>(stream, P, bits, D.num_cus, D.scratch);
   IHE_HIP(hipGetLastError());
   return IHE_OK;
 }
