@@ -333,6 +333,174 @@ __global__ __launch_bounds__(64 * kWaves) void k_cloud_mfma1(MfmaArgs A) {
 }
 
 // ---------------------------------------------------------------------------
+// The same tiles (one K-block, two row blocks) with 16-byte loads and stores:
+// lane r of a wave's column tile w (w < 4) takes word 4 r + w of 128, so that a
+// lane loads runs of four words of a column and stores runs of four words of a
+// row, 512 contiguous bytes of each row per store instruction. A stream of such
+// stores writes 6.5 TB/s where 128-byte pieces of rows write 5.2 - 5.5 TB/s
+// (rows 8 KB apart, 128 rows a workgroup), and stores are five sixths of this
+// kernel's traffic. A wave does one run of 128 words of 64 rows and ends; other
+// waves cover its latency. Columns must keep their words in runs of four:
+// unrotated, or rotated by multiples of 4.
+//
+// 80,882 targets x 1,024 samples, n = 5: 461 -> 411 us (5.8 TB/s; 381 us at the
+// rates of its reads and writes alone); 80,000 targets at NS = 512: 557 -> 456 us.
+// How it runs (launch_k1 chooses): kFew leaves the output to the infinity cache
+// (sc1 without nt) and keeps four sums per product, independent MFMAs at two
+// waves per SIMD; kFour the same with streaming stores; kTwo two sums at a time
+// (one shift's products into the higher sum, then the next), 158 registers and
+// three waves per SIMD, with the weights read from LDS and the results as whole
+// tuples until their stores. Rotated launches measured slower as kTwo (512
+// against 460 us).
+enum class Run4 { kFew, kFour, kTwo };
+
+template <bool ROT, Run4 MODE>
+__global__ __launch_bounds__(64 * kWaves)
+__attribute__((amdgpu_waves_per_eu(MODE == Run4::kTwo ? 3 : 2)))
+void k_cloud_mfma1x4(MfmaArgs A) {
+  constexpr int RB = 2;
+  constexpr uint32_t wg_per_tile = kCtWords / (kWaves * 128);
+  constexpr uint32_t rows = kMfmaRows * RB;
+  constexpr int kPolicy = MODE == Run4::kFew ? 16 : kStorePolicy;
+  __shared__ __attribute__((aligned(16))) uint32_t s_bias[rows];
+  __shared__ int4v s_a[MODE == Run4::kTwo ? RB * 2 * 64 : 1];
+  if (blockIdx.x >= A.cloud_blocks) return var_block(A.var, blockIdx.x - A.cloud_blocks);
+  const uint32_t blk = xcd_block(blockIdx.x, A.cloud_blocks), t = threadIdx.x;
+  uint32_t tile;
+  const MfmaEntry E = entry_of(A, blk / wg_per_tile, tile);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(t / 64), lane = t % 64;
+  const uint32_t h = lane / 32, r = lane % 32;
+  const MTileDev T = tile_of(E, tile);
+  const __amdgpu_buffer_rsrc_t in_r =
+      __builtin_amdgcn_make_buffer_rsrc((void *)E.in, (short)0, (int)E.in_bytes, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t out_r =
+      __builtin_amdgcn_make_buffer_rsrc((void *)E.out, (short)0, (int)E.out_bytes, kRsrcWord3);
+  if (t < rows) s_bias[t] = E.rowc[T.row_off + t];
+  uint32_t cw[16];
+  {
+    const IHE_CONSTANT uint32_t *kc = cptr(E.kcols) + T.kcol_off;
+    const u32x16v cl = *(const IHE_CONSTANT u32x16v *)kc;
+    const u32x16v chh = *(const IHE_CONSTANT u32x16v *)(kc + 16);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) cw[j] = col_word<ROT>(h ? chh[j] : cl[j], E);
+  }
+  int4v a[MODE == Run4::kTwo ? 1 : RB][2];
+  if constexpr (MODE == Run4::kTwo) {
+    for (uint32_t i = t; i < RB * 2 * 64; i += 64 * kWaves)
+      s_a[i] = E.adata[(size_t)T.a_off * 64 + i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2 * RB; ++i) a[i / 2][i % 2] = E.adata[(size_t)(T.a_off + i) * 64 + lane];
+  }
+  const uint32_t st = blk % wg_per_tile * kWaves + wave;
+  const uint32_t row_base = T.slot0 * kCtWords * 4u;
+  const bool full = T.nrows == rows;
+  __syncthreads();
+  // words n0 .. n0 + 127 of the 16 columns of this lane's half, four from n0 + 4 r on
+  const uint32_t n0 = st * 128;
+  u32x4v x[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    if constexpr (!ROT) {
+      x[j] = __builtin_bit_cast(u32x4v, __builtin_amdgcn_raw_buffer_load_b128(
+                                            in_r, cw[j] + r * 16, n0 * 4, 0));
+    } else {  // a run that wrapped past N enters negated
+      const uint32_t at = (cw[j] & 0xFFFu) + ((n0 & (kN - 1)) + 4 * r) * 4;
+      x[j] = __builtin_bit_cast(
+          u32x4v, __builtin_amdgcn_raw_buffer_load_b128(
+                      in_r, (cw[j] & ~0xFFFu) | (at & 0xFFFu), (n0 & kN) * 4, 0));
+      if (at >= kN * 4) x[j] = 0u - x[j];
+    }
+  }
+  int4v pl[4][4];  // [word of the run][plane]
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    uint32_t y[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) y[j] = x[j][w];
+    byte_planes(y, pl[w]);
+  }
+  uint32_t rbase = row_base;
+  asm volatile("" : "+s"(rbase));
+  const uint32_t word = n0 + 4 * r;
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    int16v res[4];
+    int4v a0, a1;
+    if constexpr (MODE == Run4::kTwo) {
+      a0 = s_a[2 * rb * 64 + lane];
+      a1 = s_a[(2 * rb + 1) * 64 + lane];
+    } else {
+      a0 = a[rb][0];
+      a1 = a[rb][1];
+    }
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      if constexpr (MODE == Run4::kTwo) {
+        int16v lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, pl[w][3], int16v{}, 0, 0, 0);
+        int16v hi = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, pl[w][2], lo, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, pl[w][2], int16v{}, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, pl[w][1], lo, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) hi[v] = (int)shl8_add((uint32_t)hi[v], (uint32_t)lo[v]);
+        lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, pl[w][1], int16v{}, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, pl[w][0], lo, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) hi[v] = (int)shl8_add((uint32_t)hi[v], (uint32_t)lo[v]);
+        lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, pl[w][0], int16v{}, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) hi[v] = (int)shl8_add((uint32_t)hi[v], (uint32_t)lo[v]);
+        asm volatile("" : "+v"(hi));  // stays one tuple until the stores
+        res[w] = hi;
+      } else {
+        Acc c = {};
+        mfma_kblock(a0, a1, pl[w], c);
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          res[w][v] = (int)shl8_add(shl8_add(shl8_add((uint32_t)c.s24[v], (uint32_t)c.s16[v]),
+                                             (uint32_t)c.s8[v]),
+                                    (uint32_t)c.s0[v]);
+      }
+    }
+    // bias (samples < NS) and hiding (words >= RS) of the b half
+    if (n0 >= kN && n0 - kN < E.ns) {
+      uint32_t on[4];
+#pragma unroll
+      for (int w = 0; w < 4; ++w) on[w] = word + w - kN < E.ns ? ~0u : 0u;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const u32x4v bv = *(const u32x4v *)(s_bias + 32 * rb + 8 * g + 4 * h);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int w = 0; w < 4; ++w) res[w][4 * g + q] += (int)(bv[q] & on[w]);
+      }
+    }
+    if (n0 >= kN && n0 + 127 - kN >= E.rs) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const bool keep = word + w - kN < E.rs;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) res[w][v] = keep ? res[w][v] : 0;
+      }
+    }
+    // The row's offset goes in the vector offset: a 16-byte store with a scalar
+    // offset, followed at once by a VALU write of its data registers, stored the
+    // new value in the last lanes of each 16 here (the compiler keeps the two
+    // apart only where there is no scalar offset).
+    uint32_t voff = rbase + (32 * rb + 4 * h) * kCtWords * 4u + word * 4u;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const uint32_t m = 8 * (v / 4) + (v % 4);
+      __builtin_amdgcn_raw_buffer_store_b128(
+          int4v{res[0][v], res[1][v], res[2][v], res[3][v]}, out_r,
+          full || 32 * rb + m + 4 * h < T.nrows ? voff + m * kCtWords * 4u : kDropOffset, 0,
+          kPolicy);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // NKB K-blocks (up to NKB*32 columns, wider windows), one row block per tile.
 // The tile's A operands and column words live in LDS. Within a column tile the
 // K-blocks are unrolled and each issues the next K-block's 16 loads (or the
@@ -946,10 +1114,31 @@ __device__ __forceinline__ void var_block(const VarArgs &A, uint32_t chunk, uint
 
 __global__ __launch_bounds__(256) void k_cloud_var(VarArgs A) { var_block(A, blockIdx.x); }
 
+// One-K-block tiles. Two row blocks with 4 column tiles per wave and words in
+// runs of four take the 16-byte kernel, in the way that the bytes written ask
+// for (us: dword kernel / kFew / kFour / kTwo, n = 5):
+//   rotated (NS = 512)    25 MB: 10.3 / 7.7 / 7.9 / 9.4      74 MB: 21.6 / 17.3 / 18.7 / 18.6
+//                         123 MB: 30.2 / 28.5 / 29.8 / 30.2  160 MB: 35.8 / 44.1 / 35.2 / 37.9
+//                         1,966 MB: 557 / - / 456 / 512
+//   unrotated (NS = 1024) 25 MB: 9.4 / 7.4 / 7.5 / 8.4       74 MB: 18.3 / 19.3 / 20.4 / 19.3
+//                         160 MB: 35.2 / 44.7 / 35.8 / 35.7  197 MB: 42.2 / 53.1 / 42.4 / 41.7
+//                         1,988 MB: 461 / - / 431 / 411
+// so unrotated launches of 48 to 160 MB stay on the dword kernel.
 template <bool ROT, int NTW>
-void launch_k1(hipStream_t s, int rb, dim3 grid, const MfmaArgs &A) {
-  if (rb == 2) hipLaunchKernelGGL((k_cloud_mfma1<ROT, NTW, 2>), grid, dim3(64 * kWaves), 0, s, A);
-  else hipLaunchKernelGGL((k_cloud_mfma1<ROT, NTW, 1>), grid, dim3(64 * kWaves), 0, s, A);
+void launch_k1(hipStream_t s, int rb, dim3 grid, const MfmaArgs &A, bool runs4) {
+  const dim3 block(64 * kWaves);
+  if constexpr (NTW == 4) {
+    const uint64_t mb = (uint64_t)A.cloud_blocks * (64 * 512 * 4) >> 20;  // 64 rows x 512 words per block
+    const bool few = mb < (ROT ? 128 : 48);
+    if (rb == 2 && runs4 && (ROT || few || mb >= 160)) {
+      constexpr Run4 kMany = ROT ? Run4::kFour : Run4::kTwo;
+      if (few) hipLaunchKernelGGL((k_cloud_mfma1x4<ROT, Run4::kFew>), grid, block, 0, s, A);
+      else hipLaunchKernelGGL((k_cloud_mfma1x4<ROT, kMany>), grid, block, 0, s, A);
+      return;
+    }
+  }
+  if (rb == 2) hipLaunchKernelGGL((k_cloud_mfma1<ROT, NTW, 2>), grid, block, 0, s, A);
+  else hipLaunchKernelGGL((k_cloud_mfma1<ROT, NTW, 1>), grid, block, 0, s, A);
 }
 
 template <bool ROT, int NTW>
@@ -1005,9 +1194,9 @@ void launch_rot(hipStream_t s, const MfmaShape &sh, dim3 grid, const MfmaArgs &A
     else if (sh.ntw == 16) launch_kw<ROT, 16>(s, sh.nkb, grid, A, runs4);
     else launch_kw<ROT, 8>(s, sh.nkb, grid, A, runs4);
   } else if (sh.nkb == 1) {
-    if (sh.ntw == 16) launch_k1<ROT, 16>(s, sh.rb, grid, A);
-    else if (sh.ntw == 8) launch_k1<ROT, 8>(s, sh.rb, grid, A);
-    else launch_k1<ROT, 4>(s, sh.rb, grid, A);
+    if (sh.ntw == 16) launch_k1<ROT, 16>(s, sh.rb, grid, A, runs4);
+    else if (sh.ntw == 8) launch_k1<ROT, 8>(s, sh.rb, grid, A, runs4);
+    else launch_k1<ROT, 4>(s, sh.rb, grid, A, runs4);
   } else {
     if (sh.ntw == 16) launch_kk<ROT, 16>(s, sh.nkb, grid, A);
     else if (sh.ntw == 8) launch_kk<ROT, 8>(s, sh.nkb, grid, A);
