@@ -78,7 +78,7 @@ struct VarEntry {
   const double *var_in;
   double *var_out;
   uint32_t num_out, R;
-  uint64_t rmagic;          // c / R = high 64 bits of c * rmagic (R > 1)
+  uint64_t rmagic;          // floor(2^64 / R), rounded up: div_r divides by its high word (R > 1)
 };
 
 // The variance entry of one cohort: rmagic = floor((2^64 - 1) / R) + 1 makes
