@@ -69,14 +69,15 @@ struct Keyed {
   uint32_t cohort;
   MfmaEntry e;
   uint32_t tiles;
-  // rotated 128-row tiles whose region size is a multiple of 4: their own
-  // family, launched with 16-byte staging loads
+  // rotated 128-row or one-K-block 64-row tiles whose region size is a multiple
+  // of 4: their own family, launched with 16-byte loads
   bool runs4;
 };
 
 bool same_family(const Keyed &a, const Keyed &b) {
-  return a.shape.rb == b.shape.rb && a.shape.nkb == b.shape.nkb && a.shape.ntw == b.shape.ntw &&
-         a.rot == b.rot && a.runs4 == b.runs4;
+  const bool any_ntw = a.shape.rb == kMfmaWideRb && a.shape.nkb <= kMfmaLdsNkb;  // set per launch
+  return a.shape.rb == b.shape.rb && a.shape.nkb == b.shape.nkb &&
+         (any_ntw || a.shape.ntw == b.shape.ntw) && a.rot == b.rot && a.runs4 == b.runs4;
 }
 
 VarArgs var_args(const ihe_batch *b) {
@@ -184,7 +185,7 @@ int ihe_batch_create(ihe_ctx *ctx, const ihe_cohort *cohorts, uint32_t num_cohor
       E.out = c.d_out + (size_t)s.out_base * kCtWords;
       E.out_bytes = std::min(band->num_out - s.out_base, kSegCts) * kCtWords * 4u;
       E.tile_base = s.tile_begin;
-      k.runs4 = k.rot && k.shape.rb == kMfmaWideRb && E.rs % 4 == 0;
+      k.runs4 = k.rot && (k.shape.rb == kMfmaWideRb || k.shape.rb == 2) && E.rs % 4 == 0;
       if (k.tiles) keyed.push_back(k);
     }
     if (c.d_out_var) {
@@ -217,7 +218,11 @@ int ihe_batch_create(ihe_ctx *ctx, const ihe_cohort *cohorts, uint32_t num_cohor
       first.push_back(items);
       items += keyed[j].tiles;
       item_entry.insert(item_entry.end(), keyed[j].tiles, (uint32_t)(j - i));
+      L.shape.ntw = std::max(L.shape.ntw, keyed[j].shape.ntw);
     }
+    // the launch is larger than any of its bands
+    if (!std::getenv("IHE_CLOUD_NTW") && L.shape.rb == kMfmaWideRb && L.shape.nkb <= kMfmaLdsNkb)
+      L.shape.ntw = std::max(L.shape.ntw, wide_ntw(L.shape.nkb, items));
     first.push_back(items);
     L.num_entries = (uint32_t)(j - i);
     L.num_items = items;

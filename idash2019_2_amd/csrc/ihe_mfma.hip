@@ -768,7 +768,10 @@ void k_cloud_mfmaw(MfmaArgs A) {
 // the tile writes columns 2q (lanes 0..31) and 2q + 1 (lanes 32..63); with
 // 16-byte loads (W16, where a column's words come in runs of four: unrotated,
 // or rotated by multiples of 4) it writes columns 8q..8q + 7, four words per
-// lane.
+// lane. Its time follows the K-blocks, so odd counts run as they are: n = 20 on
+// 80,882 targets (NS = 512) takes 3 instead of 4, 599 -> 522 us (32 column tiles
+// per workgroup), bound by what a workgroup waits for in turn: staged words,
+// recoding, products, stores.
 template <bool ROT, bool W16, int NTW, int NKB>
 __device__ __forceinline__ void mfmaw_lds_body(const MfmaArgs &A, uint32_t blk, int4v *s_b,
                                                uint32_t *s_raw, uint32_t *s_cw, uint32_t *s_bias,
@@ -890,7 +893,8 @@ __device__ __forceinline__ void mfmaw_lds_body(const MfmaArgs &A, uint32_t blk, 
 }
 
 template <bool ROT, bool W16, int NTW, int NKB>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ __launch_bounds__(64 * kWaves)
+__attribute__((amdgpu_waves_per_eu(NKB < 4 || (NKB == 4 && W16) ? 4 : 3)))
 void k_cloud_mfmaw_lds(MfmaArgs A) {
   __shared__ int4v s_b[NKB * 4 * 64];
   __shared__ __attribute__((aligned(16))) uint32_t s_raw[NKB * 32 * 32];
@@ -1170,15 +1174,19 @@ void launch_kk(hipStream_t s, int nkb, dim3 grid, const MfmaArgs &A) {
 template <bool ROT, bool W16, int NTW>
 void launch_kw_lds(hipStream_t s, int nkb, dim3 grid, const MfmaArgs &A) {
   const dim3 block(64 * kWaves);
-  switch ((nkb + 1) / 2) {
-    case 1: hipLaunchKernelGGL((k_cloud_mfmaw_lds<ROT, W16, NTW, 2>), grid, block, 0, s, A); break;
-    case 2: hipLaunchKernelGGL((k_cloud_mfmaw_lds<ROT, W16, NTW, 4>), grid, block, 0, s, A); break;
+  switch (nkb) {
+    case 1:
+    case 2: hipLaunchKernelGGL((k_cloud_mfmaw_lds<ROT, W16, NTW, 2>), grid, block, 0, s, A); break;
+    case 3: hipLaunchKernelGGL((k_cloud_mfmaw_lds<ROT, W16, NTW, 3>), grid, block, 0, s, A); break;
+    case 4: hipLaunchKernelGGL((k_cloud_mfmaw_lds<ROT, W16, NTW, 4>), grid, block, 0, s, A); break;
+    case 5: hipLaunchKernelGGL((k_cloud_mfmaw_lds<ROT, W16, NTW, 5>), grid, block, 0, s, A); break;
     default: hipLaunchKernelGGL((k_cloud_mfmaw_lds<ROT, W16, NTW, 6>), grid, block, 0, s, A); break;
   }
 }
 
-// tiles of nkb K-blocks run on the kernel with the next even NKB (padding
-// K-blocks carry zero weights). IHE_MFMAW_LDS: 0 = register-staged kernel,
+// tiles of nkb K-blocks run on the LDS-staged kernel of 2 to 6 K-blocks or on the
+// register-staged one with the next even NKB (padding K-blocks carry zero
+// weights). IHE_MFMAW_LDS: 0 = register-staged kernel,
 // 1 = LDS-staged with dword staging loads, else LDS-staged with 16-byte
 // staging loads where a column's words come in runs of four.
 template <bool ROT, int NTW>
@@ -1186,7 +1194,7 @@ void launch_kw(hipStream_t s, int nkb, dim3 grid, const MfmaArgs &A, bool runs4)
   const dim3 block(64 * kWaves);
   const char *e = std::getenv("IHE_MFMAW_LDS");
   const char mode = e && (e[0] == '0' || e[0] == '1') ? e[0] : '2';
-  if (mode != '0' && nkb <= 6) {
+  if (mode != '0' && nkb <= kMfmaLdsNkb) {
     if (mode == '2' && runs4) launch_kw_lds<ROT, true, NTW>(s, nkb, grid, A);
     else launch_kw_lds<ROT, false, NTW>(s, nkb, grid, A);
     return;
