@@ -109,6 +109,11 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_decrypt(const int32_t *
   }
 }
 
+// a ^ b ^ c in one instruction (truth table 0x96)
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+  return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)c, 0x96);
+}
+
 // Philox4x32-10 (Salmon et al., SC'11).
 __device__ __forceinline__ void philox(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
                                        uint32_t k0, uint32_t k1, uint32_t r[4]) {
@@ -118,9 +123,9 @@ __device__ __forceinline__ void philox(uint32_t c0, uint32_t c1, uint32_t c2, ui
     const uint64_t p0 = (uint64_t)0xD2511F53u * c0, p1 = (uint64_t)0xCD9E8D57u * c2;
     const uint32_t lo0 = (uint32_t)p0, hi0 = (uint32_t)(p0 >> 32);
     const uint32_t lo1 = (uint32_t)p1, hi1 = (uint32_t)(p1 >> 32);
-    c0 = hi1 ^ c1 ^ k0;
+    c0 = xor3(hi1, c1, k0);
     c1 = lo1;
-    c2 = hi0 ^ c3 ^ k1;
+    c2 = xor3(hi0, c3, k1);
     c3 = lo0;
     k0 += 0x9E3779B9u;
     k1 += 0xBB67AE85u;
@@ -148,27 +153,43 @@ __device__ __forceinline__ int32_t noise_sample(uint64_t u, const uint64_t *__re
   return (u & 1) ? -(int32_t)k : (int32_t)k;
 }
 
-// The same sample, the search started from the bucket index (build_noise_lut):
-// three steps where the bucket spans at most 7 entries (all but the tails
-// beyond about 3.5 sigma), the full eleven from the bucket's low end otherwise.
-__device__ __forceinline__ int32_t noise_sample_lut(uint64_t u, const uint64_t *table,
-                                                    const uint32_t *lut) {
-  const uint64_t m = u >> 1;
-  const uint32_t e = lut[m >> (63 - kNoiseLutBits)];
-  uint32_t k = e & 0xFFFFu;
-  auto step_to = [&](uint32_t step) {
-    const uint32_t nk = k + step;
-    const uint64_t tv = table[min(nk, IHE_NOISE_TABLE_LEN - 1) - 1];
-    k = nk <= IHE_NOISE_TABLE_LEN - 1 && tv <= m ? nk : k;
-  };
-  if ((e >> 16) <= 7) {
+// The same samples of four words at once, each search started from its bucket
+// (lut: low end, and entries in the bucket up to kNoiseLutMany, from
+// build_noise_lut). Three steps do where every bucket of the wave spans at most
+// 7 entries; two more are taken where one spans up to 30 (beyond about 3.2
+// sigma, one wave in four), the remaining six beyond 3.6 sigma (one in sixteen).
+// The four words take them together, so that their LDS reads overlap, and
+// kNoisePad entries above every m follow the table in place of a bound.
+constexpr uint32_t kNoiseLutMany = 31;
+constexpr uint32_t kNoisePad = 32;
+__device__ __forceinline__ void noise_sample4(const uint64_t u[4], const uint64_t *table,
+                                              const uint16_t *lut, uint32_t e[4]) {
+  static_assert(IHE_NOISE_TABLE_LEN < 2048, "the low end takes 11 bits");
+  uint32_t k[4], many = 0;
 #pragma unroll
-    for (uint32_t step = 4; step > 0; step >>= 1) step_to(step);
-  } else {
-#pragma unroll
-    for (uint32_t step = 1024; step > 0; step >>= 1) step_to(step);
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t l = lut[(uint32_t)(u[i] >> (64 - kNoiseLutBits))];
+    k[i] = l & 2047u;
+    many = max(many, l >> 11);
   }
-  return (u & 1) ? -(int32_t)k : (int32_t)k;
+  auto step4 = [&](uint32_t step, bool pad) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t at = pad ? k[i] + step : min(k[i] + step, IHE_NOISE_TABLE_LEN);
+      k[i] += table[at - 1] <= (u[i] >> 1) ? step : 0;
+    }
+  };
+  if (__builtin_expect(__any(many > 7), 0)) {
+    if (__any(many >= kNoiseLutMany))
+      for (uint32_t step = 1024; step > 16; step >>= 1) step4(step, false);
+    step4(16, true);
+    step4(8, true);
+  }
+  step4(4, true);
+  step4(2, true);
+  step4(1, true);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) e[i] = (u[i] & 1) ? 0u - k[i] : k[i];
 }
 
 // ---------------------------------------------------------------------------
@@ -579,51 +600,74 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_encrypt(EncryptParams P
 // one counter per two words, e sampled from the CDF table), and the variance.
 // k_ring_mfma<true> then adds a*s to b. Persistent workgroups copy the CDF
 // table to LDS (its searches are scattered reads) and take ciphertexts in
-// turn, a thread four words j..j+3 of each.
-__global__ __launch_bounds__(256) void k_encrypt_ae(EncryptParams P) {
+// turn, a thread four words j..j+3 of each. VALU-bound (54 multiply-adds of
+// Philox, four searches and four messages a thread), so searches and messages
+// are selects instead of branches. Six workgroups fit a CU by registers and by
+// LDS (bucket index in 16 bits), and the grid is that many: the grid of eight
+// before left its last quarter to a second, half-empty wave of workgroups. At
+// seven or eight a CU the registers spill (encryption of 48,552 ciphertexts: 268
+// us at 5 and 6, 299 at 7, 341 at 8; 314 with branches and a grid of eight).
+constexpr uint32_t kAeBlocks = 6;
+__global__ __launch_bounds__(256, kAeBlocks) void k_encrypt_ae(EncryptParams P) {
   typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
-  __shared__ uint64_t s_table[IHE_NOISE_TABLE_LEN];
-  __shared__ uint32_t s_lut[1u << kNoiseLutBits];
-  for (uint32_t t = threadIdx.x; t < IHE_NOISE_TABLE_LEN; t += 256) s_table[t] = P.table[t];
-  for (uint32_t t = threadIdx.x; t < (1u << kNoiseLutBits); t += 256) s_lut[t] = P.lut[t];
+  constexpr int kRsrc3 = 0x00020000;  // raw buffer descriptor, dword 3
+  __shared__ uint64_t s_table[IHE_NOISE_TABLE_LEN + kNoisePad];
+  __shared__ uint16_t s_lut[1u << kNoiseLutBits];
+  for (uint32_t t = threadIdx.x; t < IHE_NOISE_TABLE_LEN + kNoisePad; t += 256)
+    s_table[t] = t < IHE_NOISE_TABLE_LEN ? P.table[t] : ~0ull;
+  for (uint32_t t = threadIdx.x; t < (1u << kNoiseLutBits); t += 256) {
+    const uint32_t l = P.lut[t];
+    s_lut[t] = (uint16_t)((l & 0xFFFFu) | min(l >> 16, kNoiseLutMany) << 11);
+  }
   __syncthreads();
   const uint32_t q = threadIdx.x;
+  // word 4 q's region and sample; the next words follow in the same region or
+  // at the start of the next one
+  const uint32_t rr0 = (uint32_t)(((uint64_t)(4 * q) * P.rs_recip) >> 32), sj0 = 4 * q - rr0 * P.rs;
   for (uint32_t ct = blockIdx.x; ct < P.num_cts; ct += gridDim.x) {
     int32_t *a = P.out + (size_t)ct * kCtWords;
     // The genotype bytes of this thread's four b words (setScore) are loaded
-    // first, so that their latency runs under the Philox rounds below.
+    // first, so that their latency runs under the Philox rounds below. Words
+    // without a message load nothing and match no genotype.
     int32_t g[4] = {0, 0, 0, 0};
-    uint32_t val[4] = {0, 0, 0, 0};
-    bool has[4] = {false, false, false, false};
+    uint32_t val[4] = {3, 3, 3, 3};
     if (P.geno) {
+      const uint32_t col0 = ct * P.R, tag0 = col0 / 3;
+      const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<int8_t *>(P.geno + (size_t)tag0 * P.ns), 0, 0x7FFFFFFF, kRsrc3);
+      uint32_t rr = rr0, sj = sj0;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const uint32_t j = 4 * q + u;
-        const uint32_t rr = (uint32_t)(((uint64_t)j * P.rs_recip) >> 32), sj = j - rr * P.rs;
-        const uint32_t bidx = ct * P.R + rr, tag = bidx / 3;
-        has[u] = rr < P.R && sj < P.ns && bidx < P.num_cols;
-        val[u] = bidx - 3 * tag;
-        if (has[u]) g[u] = P.geno[(size_t)tag * P.ns + sj];
+        const uint32_t col = col0 - 3 * tag0 + rr, tag = col * 683 >> 11;  // col / 3, col < 2,048
+        const bool has = rr < P.R && sj < P.ns && col0 + rr < P.num_cols;
+        const uint32_t off = has ? tag * P.ns + sj : ~0u;
+        val[u] = has ? col - 3 * tag : 3u;
+        g[u] = (int8_t)__builtin_amdgcn_raw_buffer_load_b8(rows, off, 0, 0);
+        ++sj;
+        rr += sj == P.rs;
+        sj = sj == P.rs ? 0 : sj;
       }
     }
     uint32_t r[4];
     philox(q, ct, 0, 0, P.seed_lo, P.seed_hi, r);
     *(u32x4v *)(a + 4 * q) = u32x4v{r[0], r[1], r[2], r[3]};
-    uint32_t b[4];
+    uint64_t w[4];
 #pragma unroll
     for (int pr = 0; pr < 2; ++pr) {
       philox(2 * q + pr, ct, 1, 0, P.seed_lo, P.seed_hi, r);
-      b[2 * pr] = (uint32_t)noise_sample_lut((uint64_t)r[0] | ((uint64_t)r[1] << 32), s_table, s_lut);
-      b[2 * pr + 1] =
-          (uint32_t)noise_sample_lut((uint64_t)r[2] | ((uint64_t)r[3] << 32), s_table, s_lut);
+      w[2 * pr] = (uint64_t)r[0] | ((uint64_t)r[1] << 32);
+      w[2 * pr + 1] = (uint64_t)r[2] | ((uint64_t)r[3] << 32);
     }
+    uint32_t b[4];
+    noise_sample4(w, s_table, s_lut, b);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if (!has[u]) continue;
-      if (g[u] == 0 || g[u] == 1 || g[u] == 2) {
-        if ((uint32_t)g[u] == val[u]) b[u] += kOne;
-      } else {
-        b[u] += val[u] == 0 ? kNan[0] : (val[u] == 1 ? kNan[1] : kNan[2]);
+    for (int u = 0; u < 4; ++u) b[u] += (uint32_t)g[u] == val[u] ? kOne : 0u;
+    if (max(max((uint32_t)g[0], (uint32_t)g[1]), max((uint32_t)g[2], (uint32_t)g[3])) > 2) {
+      // missing genotypes (a word without a message has g = 0)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t t = val[u] == 0 ? kNan[0] : (val[u] == 1 ? kNan[1] : kNan[2]);
+        b[u] += (uint32_t)g[u] > 2 ? t : 0u;
       }
     }
     *(u32x4v *)(a + kN + 4 * q) = u32x4v{b[0], b[1], b[2], b[3]};
@@ -785,7 +829,7 @@ int ihe_encrypt(ihe_ctx *ctx, const ihe_key *key, const ihe_layout *layout, uint
     const RingParams D{d_out, nullptr, d_out, P.num_cts, NS, 0, 0, nullptr};
     ScopedTimer t(ctx, IHE_TIMER_ENCRYPT);
     static_assert(kN / 4 == 256, "a thread per four words of a ciphertext");
-    hipLaunchKernelGGL(k_encrypt_ae, dim3(std::min<uint32_t>(P.num_cts, (uint32_t)ctx->num_cus * 8)),
+    hipLaunchKernelGGL(k_encrypt_ae, dim3(std::min<uint32_t>(P.num_cts, (uint32_t)ctx->num_cus * kAeBlocks)),
                        dim3(256), 0, ctx->stream, P);
     launch_ring<true>(ctx->stream, D, key->bits, (uint32_t)ctx->num_cus, ctx->d_ring_queue);
     IHE_HIP(hipGetLastError());
