@@ -939,30 +939,51 @@ uint32_t env_u32(const char *name, uint32_t dflt, uint32_t lo, uint32_t hi) {
   return dflt;
 }
 
-// Number of tiles `shape` cuts the outputs into (0 when a row does not fit).
-uint32_t count_tiles(uint32_t num_out, const MfmaShape &shape, const HostBand &H) {
+// What count_tiles needs for every shape of a band: each output's group, and the
+// groups' columns as small numbers to mark (the columns themselves where they
+// are dense, else their ranks).
+struct ColumnIds {
+  std::vector<uint32_t> group_of, id, tile_of;
+  ColumnIds(uint32_t num_out, const HostBand &H) : group_of(num_out), id(H.gcol) {
+    for (uint32_t g = 0; g < H.hg.size(); ++g)
+      for (uint32_t i = 0; i < H.hg[g].nout; ++i) group_of[H.gout[H.hg[g].out_begin + i]] = g;
+    size_t n = H.has_cols ? (size_t)H.max_bidx + 1 : 0;
+    if (n > 16 * id.size() + 4096) {
+      std::vector<uint32_t> sorted(id);
+      std::sort(sorted.begin(), sorted.end());
+      sorted.erase(std::unique(sorted.begin(), sorted.end()), sorted.end());
+      for (uint32_t &c : id)
+        c = (uint32_t)(std::lower_bound(sorted.begin(), sorted.end(), c) - sorted.begin());
+      n = sorted.size();
+    }
+    tile_of.resize(n);
+  }
+};
+
+// Number of tiles `shape` cuts the outputs into (0 when a row does not fit). The
+// shape search runs it for up to seven shapes, so a tile's distinct columns are
+// counted by marks instead of merging sorted lists (14,993 targets of 99
+// columns: the band compiles in 154 ms instead of 203 ms).
+uint32_t count_tiles(uint32_t num_out, const MfmaShape &shape, const HostBand &H, ColumnIds &C) {
   const uint32_t rows = kMfmaRows * (uint32_t)shape.rb, budget = 32 * (uint32_t)shape.nkb;
-  std::vector<uint32_t> og(num_out);
-  for (uint32_t g = 0; g < H.hg.size(); ++g)
-    for (uint32_t i = 0; i < H.hg[g].nout; ++i) og[H.gout[H.hg[g].out_begin + i]] = g;
-  std::vector<uint32_t> u, merged;
+  std::fill(C.tile_of.begin(), C.tile_of.end(), UINT32_MAX);
   uint32_t tiles = 0;
   for (uint32_t o = 0; o < num_out;) {
     const uint32_t o0 = o;
-    u.clear();
-    uint32_t last_g = UINT32_MAX;
+    uint32_t last_g = UINT32_MAX, n = 0;  // n: columns of the tile
     while (o < num_out && o - o0 < rows) {
-      const uint32_t g = og[o];
+      const uint32_t g = C.group_of[o];
       if (g != last_g) {
         const HostGroup &hg = H.hg[g];
-        merged.clear();
-        std::set_union(u.begin(), u.end(), H.gcol.begin() + hg.col_begin,
-                       H.gcol.begin() + hg.col_begin + hg.ncol, std::back_inserter(merged));
-        if (merged.size() > budget) {
+        for (uint32_t i = 0; i < hg.ncol; ++i) {
+          uint32_t &t = C.tile_of[C.id[hg.col_begin + i]];
+          n += t != tiles;
+          t = tiles;
+        }
+        if (n > budget) {
           if (o == o0) return 0;
           break;
         }
-        u.swap(merged);
         last_g = g;
       }
       ++o;
@@ -991,13 +1012,14 @@ int pick_ntw(int rb, int nkb, uint32_t tiles) {
 // K-blocks, 0.98 ms for 128 x 8, against 1.01 ms for 32 x 5). The kernel
 // autotuner (ihe_band_create_tuned) refines this choice by measurement.
 bool pick_mfma_shape(uint32_t num_out, HostBand &H, MfmaShape &shape) {
+  ColumnIds ids(num_out, H);
   if (const char *e = std::getenv("IHE_CLOUD_SHAPE")) {
     int rb = 0, nkb = 0;
     if (std::sscanf(e, "%d,%d", &rb, &nkb) == 2 &&
         (rb == 1 || (rb == 2 && nkb == 1) || rb == kMfmaWideRb) && nkb >= 1 &&
         nkb <= (int)kMfmaMaxNkb) {
       shape = {rb, nkb, 4};
-      const uint32_t t = count_tiles(num_out, shape, H);
+      const uint32_t t = count_tiles(num_out, shape, H, ids);
       shape.ntw = pick_ntw(rb, nkb, t);
       return t > 0;
     }
@@ -1013,7 +1035,7 @@ bool pick_mfma_shape(uint32_t num_out, HostBand &H, MfmaShape &shape) {
   double best = 0;
   bool found = false;
   for (MfmaShape &c : cands) {
-    const uint32_t t = count_tiles(num_out, c, H);
+    const uint32_t t = count_tiles(num_out, c, H, ids);
     if (t == 0) continue;
     c.ntw = pick_ntw(c.rb, c.nkb, t);
     H.candidates.push_back(c);
@@ -1151,8 +1173,8 @@ int plan_band(const ihe_layout *layout, uint32_t num_in_cts, const ihe_model_csr
   }
   if (mode == kModeMfma) {
     MfmaShape shape;
-    const bool ok = force_shape ? (shape = *force_shape, count_tiles(model->num_outputs, shape, H) > 0)
-                          : pick_mfma_shape(model->num_outputs, H, shape);
+    if (force_shape) shape = *force_shape;
+    const bool ok = force_shape || pick_mfma_shape(model->num_outputs, H, shape);
     if (!ok || !layout_mfma(model->num_outputs, shape, H)) {
       if (variant == IHE_VARIANT_MFMA)
         return fail(IHE_ERR_UNSUPPORTED, "an MFMA tile needs more than 256 distinct columns");
