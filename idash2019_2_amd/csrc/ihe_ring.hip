@@ -602,13 +602,20 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_encrypt(EncryptParams P
 // table to LDS (its searches are scattered reads) and take ciphertexts in
 // turn, a thread four words j..j+3 of each. VALU-bound (54 multiply-adds of
 // Philox, four searches and four messages a thread), so searches and messages
-// are selects instead of branches. Six workgroups fit a CU by registers and by
-// LDS (bucket index in 16 bits), and the grid is that many: the grid of eight
-// before left its last quarter to a second, half-empty wave of workgroups. At
-// seven or eight a CU the registers spill (encryption of 48,552 ciphertexts: 268
-// us at 5 and 6, 299 at 7, 341 at 8; 314 with branches and a grid of eight).
-constexpr uint32_t kAeBlocks = 6;
-__global__ __launch_bounds__(256, kAeBlocks) void k_encrypt_ae(EncryptParams P) {
+// are selects instead of branches. As many workgroups share a CU as registers
+// and LDS (bucket index in 16 bits) allow, and the grid is that many: the grid
+// of eight before left its last quarter to a second, half-empty wave of
+// workgroups (48,552 ciphertexts, encryption: 314 us with branches and a grid of
+// eight; 268 us at 5 and 6 a CU, 299 at 7 and 341 at 8, where registers spill).
+//
+// ONE is for one region (NS > 512): a ciphertext is one column, its tag and
+// value are scalars and a word's genotype byte lies at the word's own offset,
+// which saves 40 of some 300 vector instructions and leaves registers for seven
+// workgroups: 261.3 -> 252.4 us (253.9 at six).
+template <bool ONE>
+constexpr uint32_t kAeBlocks = ONE ? 7 : 6;
+template <bool ONE>
+__global__ __launch_bounds__(256, kAeBlocks<ONE>) void k_encrypt_ae(EncryptParams P) {
   typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
   constexpr int kRsrc3 = 0x00020000;  // raw buffer descriptor, dword 3
   __shared__ uint64_t s_table[IHE_NOISE_TABLE_LEN + kNoisePad];
@@ -631,7 +638,16 @@ __global__ __launch_bounds__(256, kAeBlocks) void k_encrypt_ae(EncryptParams P) 
     // without a message load nothing and match no genotype.
     int32_t g[4] = {0, 0, 0, 0};
     uint32_t val[4] = {3, 3, 3, 3};
-    if (P.geno) {
+    if (ONE && P.geno) {
+      const uint32_t tag = ct / 3;
+      const __amdgpu_buffer_rsrc_t row = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<int8_t *>(P.geno + (size_t)tag * P.ns), 0, P.ns, kRsrc3);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        val[u] = 4 * q + u < P.ns ? ct - 3 * tag : 3u;
+        g[u] = (int8_t)__builtin_amdgcn_raw_buffer_load_b8(row, 4 * q + u, 0, 0);
+      }
+    } else if (P.geno) {
       const uint32_t col0 = ct * P.R, tag0 = col0 / 3;
       const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
           const_cast<int8_t *>(P.geno + (size_t)tag0 * P.ns), 0, 0x7FFFFFFF, kRsrc3);
@@ -829,8 +845,12 @@ int ihe_encrypt(ihe_ctx *ctx, const ihe_key *key, const ihe_layout *layout, uint
     const RingParams D{d_out, nullptr, d_out, P.num_cts, NS, 0, 0, nullptr};
     ScopedTimer t(ctx, IHE_TIMER_ENCRYPT);
     static_assert(kN / 4 == 256, "a thread per four words of a ciphertext");
-    hipLaunchKernelGGL(k_encrypt_ae, dim3(std::min<uint32_t>(P.num_cts, (uint32_t)ctx->num_cus * kAeBlocks)),
-                       dim3(256), 0, ctx->stream, P);
+    const auto launch_ae = [&](void (*ae)(EncryptParams), uint32_t blocks) {
+      hipLaunchKernelGGL(ae, dim3(std::min<uint32_t>(P.num_cts, (uint32_t)ctx->num_cus * blocks)),
+                         dim3(256), 0, ctx->stream, P);
+    };
+    if (P.R == 1) launch_ae(k_encrypt_ae<true>, kAeBlocks<true>);
+    else launch_ae(k_encrypt_ae<false>, kAeBlocks<false>);
     launch_ring<true>(ctx->stream, D, key->bits, (uint32_t)ctx->num_cus, ctx->d_ring_queue);
     IHE_HIP(hipGetLastError());
     return IHE_OK;
