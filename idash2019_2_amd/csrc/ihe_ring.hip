@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "ihe_internal.h"
+#include "ihe_rules.h"
 
 // Work counters of ihe_decrypt_noalloc: the ring kernel's per-XCD item
 // counters and its count of finished workgroups, in a file-scope device array
@@ -259,7 +260,7 @@ __device__ __forceinline__ uint32_t u_byte(uint32_t y, const uint32_t *kw) {
   return bit * ((y > kN) != NEG ? 0xFFu : 1u);
 }
 
-constexpr uint32_t kRuns = 2 * kN - 16;  // 16-byte runs of u that B operands are made of
+static_assert(kRuns == 2 * kN - 16, "16-byte runs of u that B operands are made of");
 constexpr uint32_t kRingThreads = 512, kRingWaves = kRingThreads / 64;
 
 struct RingLds {
@@ -405,7 +406,7 @@ void k_ring_mfma(RingParams P, KeyBits key) {
     const bool active = nt0 * 32 < lim, full = rows == 32, more = next < it_end;
     const __amdgpu_buffer_rsrc_t nr = in_rsrc(more ? next : item, more);
     const uint32_t nvo = a_off(more ? next : item);
-    const int4v *const bl = (const int4v *)S.u + (kN - 1 - 32 * nt0 - c + 16 * h);
+    const int4v *const bl = (const int4v *)S.u + ring_run(nt0, h, c);
     int16v acc[TPW];
     // plane p's K-blocks; hook(ks) issues the step's share of other work, and a
     // scheduling barrier keeps it there
@@ -414,7 +415,8 @@ void k_ring_mfma(RingParams P, KeyBits key) {
       auto slot = [](int d) { return (d + 32 * kSlots) % kSlots; };
       int4v w[kSlots], a[3];
 #pragma unroll
-      for (int t = 0; t < TPW; ++t) w[t] = bl[-32 * t];
+      for (int t = 0; t < TPW; ++t)
+        w[t] = bl[kRingWordTiles % TPW ? 32 * ((int)nt0 - (int)ring_operand_tile(nt0 + t)) : -32 * t];
       w[slot(-1)] = bl[32];
       a[0] = *(const int4v *)(ra0 + p * 32768);
       a[1] = *(const int4v *)(ra1 + p * 32768 + 1024);
