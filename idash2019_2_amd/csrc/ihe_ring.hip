@@ -270,7 +270,17 @@ struct RingLds {
 };
 static_assert(sizeof(RingLds) <= 160 * 1024, "one workgroup's LDS");
 
-template <bool ENC, int TPW>
+// NT: a-words by streaming (nt) loads, for decryptions of kRingStreamCts
+// ciphertexts and more. Their a-words (4 KB each) pass through the 256 MB
+// infinity cache without being found there again, and loads that leave lines
+// behind made 242,646 x 256 take 298 us and x 160 271 us; streaming they take 280
+// and 248 us (three inputs in turn: 294 and 266; the kernel of 256-word items: 290
+// and 260). Below it they find part of an input that was decrypted before:
+// 45,011 x 256 takes 55.6 us plain and 61.7 us streaming, 100,000 x 256 128 and
+// 122 us. At four tiles a wave the MFMAs hide either (242,646 x 1,024: 742, 743 us).
+constexpr uint32_t kRingStreamCts = 3u << 15;
+
+template <bool ENC, int TPW, bool NT = false>
 __global__ __launch_bounds__(kRingThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_ring_mfma(RingParams P, KeyBits key) {
   typedef int int4v __attribute__((ext_vector_type(4)));
@@ -305,7 +315,8 @@ void k_ring_mfma(RingParams P, KeyBits key) {
   };
   auto a_off = [&](uint32_t it) { return min(lr, rows_of(it) - 1) * kCtBytes + lc * 16; };
   auto load_a = [&](const __amdgpu_buffer_rsrc_t &R, uint32_t vo, int i) {
-    q[i] = __builtin_bit_cast(u32x4v, __builtin_amdgcn_raw_buffer_load_b128(R, vo + 256 * i, 0, 0));
+    q[i] = __builtin_bit_cast(u32x4v, __builtin_amdgcn_raw_buffer_load_b128(R, vo + 256 * i, 0,
+                                                                          NT ? 2 : 0));
   };
   auto put = [&](int p, int i) { wp[p * 8192 + i * 512] = q[i][p]; };
   // piece i: four words -> their digits by plane; planes 3 and 2 written
@@ -737,11 +748,16 @@ void launch_ring(hipStream_t stream, RingParams P, const KeyBits &key, uint32_t 
   P.num_items = groups * P.col_groups;
   const dim3 grid(std::min<uint32_t>((num_cus + 7) / 8 * 8, (P.num_items + 7) / 8 * 8));
   const dim3 block(kRingThreads);
+  // encryption reads back the a-words that it has just written
+  const bool nt = !ENC && P.num_cts >= kRingStreamCts;
+  const auto launch = [&](void (*plain)(RingParams, KeyBits), void (*stream_a)(RingParams, KeyBits)) {
+    hipLaunchKernelGGL(nt ? stream_a : plain, grid, block, 0, stream, P, key);
+  };
   switch (tpw) {
-    case 1: hipLaunchKernelGGL((k_ring_mfma<ENC, 1>), grid, block, 0, stream, P, key); break;
-    case 2: hipLaunchKernelGGL((k_ring_mfma<ENC, 2>), grid, block, 0, stream, P, key); break;
-    case 3: hipLaunchKernelGGL((k_ring_mfma<ENC, 3>), grid, block, 0, stream, P, key); break;
-    default: hipLaunchKernelGGL((k_ring_mfma<ENC, 4>), grid, block, 0, stream, P, key); break;
+    case 1: launch(k_ring_mfma<ENC, 1>, k_ring_mfma<ENC, 1, !ENC>); break;
+    case 2: launch(k_ring_mfma<ENC, 2>, k_ring_mfma<ENC, 2, !ENC>); break;
+    case 3: launch(k_ring_mfma<ENC, 3>, k_ring_mfma<ENC, 3, !ENC>); break;
+    default: launch(k_ring_mfma<ENC, 4>, k_ring_mfma<ENC, 4>); break;
   }
 }
 
