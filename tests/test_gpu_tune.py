@@ -1,0 +1,27 @@
+"""The autotuner times a shape's column-tile counts at one clock: after the pause
+in which a shape is compiled and uploaded, the card's clock swings for some 20 ms.
+The three counts of 128 x 6 tiles lie within 10 % of each other at a steady clock
+(40,000 targets of 50 tags: 378, 380 and 405 us); timed one after another, two
+launches each, right after that pause, the table had them 50 to 70 % apart. The
+bound lies between the two."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def test_counts_are_timed_at_one_clock(engine):
+    targets, n = 40000, 50
+    tags = targets // 5
+    rng = np.random.default_rng(1)
+    lo = np.minimum(np.arange(targets) // 5, tags - n)
+    ib = (np.repeat(3 * lo, 3)[:, None] + np.arange(3 * n)).astype(np.uint32)
+    rp = np.arange(3 * targets + 1, dtype=np.uint32) * (3 * n)
+    w = rng.integers(-100, 100, ib.size, dtype=np.int16).astype(np.int32)
+    d_in = engine.to_device(rng.integers(-(1 << 31), 1 << 31, (3 * tags, 2, 1024), dtype=np.int32))
+    d_out = engine.empty((3 * targets, 2, 1024), np.int32)
+    band, table = engine.band_tuned(1024, 3 * tags, rp, ib.ravel(), w, d_in, d_out, reps=2)
+    band.free()
+    ms = {c: t for rows, kb, c, t in table if (rows, kb) == (128, 6)}
+    assert set(ms) == {8, 16, 32}
+    assert max(ms.values()) < 1.25 * min(ms.values()), ms
