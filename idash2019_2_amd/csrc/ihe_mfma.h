@@ -4,6 +4,7 @@
 #pragma once
 
 #include "ihe_internal.h"
+#include "ihe_rules.h"
 
 namespace ihe {
 
@@ -56,21 +57,6 @@ struct MfmaShape {
   int nkb = 1;  // K-blocks per tile
   int ntw = 4;  // 32-word column tiles per wave (per workgroup for rb 4)
 };
-
-// Column tiles per workgroup of the LDS-staged 128-row kernel (up to kMfmaLdsNkb
-// K-blocks) for a launch of `tiles` tiles: few column tiles make enough
-// workgroups of a small launch, many save a large one the start of each (us at
-// 8 / 16 / 32):
-//   n = 10, 2 K-blocks, NS = 1024   60 tiles 16 / 20 / 35    119: 33 / 30 / 35    1,900: 479 / 478 / 494
-//   n = 20, 3 K-blocks, NS = 512    60: 19 / 26 / 48    238: 62 / 63 / 73    952: 300 / 285 / 277
-//                                   1,900: 591 / 565 / 535
-//   n = 50, 6 K-blocks, NS = 100    60: 32 / 44 / 84    119: 61 / 61 / 84    476: 216 / 217 / 224
-//                                   952: 443 / 428 / 435    1,907: 889 / 861 / 846
-constexpr int kMfmaLdsNkb = 6;
-inline int wide_ntw(int nkb, uint32_t tiles) {
-  if (tiles < (nkb <= 2 ? 100u : 200u)) return 8;
-  return nkb > 2 && tiles >= 900 ? 32 : 16;
-}
 
 // Workgroups per tile of a shape (a ciphertext has kCtWords / 32 column tiles).
 inline uint32_t mfma_wg_per_tile(const MfmaShape &s) {
