@@ -68,7 +68,7 @@ struct Keyed {
   bool rot;
   uint32_t cohort;
   MfmaEntry e;
-  uint32_t tiles;
+  uint32_t tiles, band_tiles;
   // rotated 128-row or one-K-block 64-row tiles whose region size is a multiple
   // of 4: their own family, launched with 16-byte loads
   bool runs4;
@@ -168,6 +168,7 @@ int ihe_batch_create(ihe_ctx *ctx, const ihe_cohort *cohorts, uint32_t num_cohor
       k.rot = L.num_regions > 1;
       k.cohort = i;
       k.tiles = s.tile_end - s.tile_begin;
+      k.band_tiles = band->num_tiles;
       MfmaEntry &E = k.e;
       E = {};
       E.tiles = band->d_mtiles;
@@ -212,17 +213,17 @@ int ihe_batch_create(ihe_ctx *ctx, const ihe_cohort *cohorts, uint32_t num_cohor
     size_t j = i;
     ihe_batch::Launch L{keyed[i].shape, keyed[i].rot, (uint32_t)entries.size(), 0,
                         (uint32_t)first.size(), 0, (uint32_t)item_entry.size(), keyed[i].runs4};
-    uint32_t items = 0;
+    uint32_t items = 0, band_tiles = 0;
     for (; j < keyed.size() && same_family(keyed[i], keyed[j]); ++j) {
       entries.push_back(keyed[j].e);
       first.push_back(items);
       items += keyed[j].tiles;
       item_entry.insert(item_entry.end(), keyed[j].tiles, (uint32_t)(j - i));
       L.shape.ntw = std::max(L.shape.ntw, keyed[j].shape.ntw);
+      band_tiles = std::max(band_tiles, keyed[j].band_tiles);
     }
-    // the launch is larger than any of its bands
     if (!std::getenv("IHE_CLOUD_NTW") && L.shape.rb == kMfmaWideRb && L.shape.nkb <= kMfmaLdsNkb)
-      L.shape.ntw = std::max(L.shape.ntw, wide_ntw(L.shape.nkb, items));
+      L.shape.ntw = family_ntw(L.shape.nkb, L.shape.ntw, band_tiles, items);
     first.push_back(items);
     L.num_entries = (uint32_t)(j - i);
     L.num_items = items;

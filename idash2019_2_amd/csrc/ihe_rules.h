@@ -62,4 +62,13 @@ constexpr int wide_ntw(int nkb, uint32_t tiles) {
   return nkb > 2 && tiles >= many ? 32 : 16;
 }
 
+// Column tiles of a batch's 128-row family of `tiles` tiles, whose bands run up
+// to `most` by themselves, the largest of them with `band_tiles` tiles. A launch
+// no larger than a band keeps the band's count (the autotuner may have measured
+// it); a larger one goes by its own tiles.
+constexpr int family_ntw(int nkb, int most, uint32_t band_tiles, uint32_t tiles) {
+  const int rule = wide_ntw(nkb, tiles);
+  return tiles > band_tiles && rule > most ? rule : most;
+}
+
 }  // namespace ihe

@@ -2,6 +2,7 @@
 // form that they are used in. Prints the first value that is out of place and
 // ends with 1; 0 when all hold.
 #include <cstdio>
+#include <initializer_list>
 
 #include "ihe_rules.h"
 
@@ -49,4 +50,23 @@ static int column_tiles() {
   return 0;
 }
 
-int main() { return ring_operands() || column_tiles(); }
+// A batch keeps the count that a band of its own size was tuned to; a launch of
+// more tiles than its bands goes by the rule, but not below them.
+static int family_column_tiles() {
+  for (int nkb = 2; nkb <= kMfmaLdsNkb; ++nkb)
+    for (int most : {8, 16, 32})
+      for (uint32_t band : {1u, 119u, 378u, 1907u}) {
+        if (family_ntw(nkb, most, band, band) != most)
+          return std::printf("%d K-blocks: a launch of its band's %u tiles runs %d instead of %d\n",
+                             nkb, band, family_ntw(nkb, most, band, band), most), 1;
+        for (uint32_t tiles : {band + 1, 2 * band, 16 * band}) {
+          const int rule = wide_ntw(nkb, tiles), want = tiles == band || rule < most ? most : rule;
+          if (family_ntw(nkb, most, band, tiles) != want)
+            return std::printf("%d K-blocks: %u tiles of %u-tile bands run %d instead of %d\n", nkb,
+                               tiles, band, family_ntw(nkb, most, band, tiles), want), 1;
+        }
+      }
+  return 0;
+}
+
+int main() { return ring_operands() || column_tiles() || family_column_tiles(); }
