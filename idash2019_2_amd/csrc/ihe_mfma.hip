@@ -473,7 +473,8 @@ void k_cloud_mfma1x4(MfmaArgs A) {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
 #pragma unroll
-          for (int w = 0; w < 4; ++w) res[w][4 * g + q] += (int)(bv[q] & on[w]);
+          for (int w = 0; w < 4; ++w)
+            res[w][4 * g + q] = add_words(res[w][4 * g + q], bv[q] & on[w]);
       }
     }
     if (n0 >= kN && n0 + 127 - kN >= E.rs) {

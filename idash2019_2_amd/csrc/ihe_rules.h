@@ -6,6 +6,10 @@
 
 namespace ihe {
 
+// A result word (an accumulator's int32) plus a torus word, mod 2^32: torus words
+// wrap as a matter of course, which a signed sum may not.
+constexpr int32_t add_words(int32_t a, uint32_t b) { return (int32_t)((uint32_t)a + b); }
+
 // Ring kernel: word tiles of 32 words (32 of them to a polynomial), and the
 // 16-byte runs of u that its B operands are made of.
 constexpr uint32_t kRingWordTiles = 32;

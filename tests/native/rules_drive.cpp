@@ -8,6 +8,11 @@
 
 using namespace ihe;
 
+// Sums of torus words wrap (an overflowing signed sum is no constant expression,
+// so it would not compile here).
+static_assert(add_words(INT32_MAX, 1u) == INT32_MIN && add_words(INT32_MIN, 0x80000000u) == 0 &&
+              add_words(-1, 1u) == 0 && add_words(INT32_MIN, 0xFFFFFFFFu) == INT32_MAX, "mod 2^32");
+
 // Ring kernel: every B operand that an active wave reads, at every number of
 // tiles a wave, lies in the table of runs, and tiles that give results read
 // their own.
