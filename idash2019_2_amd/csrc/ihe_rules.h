@@ -32,29 +32,32 @@ constexpr uint32_t ring_run(uint32_t nt, uint32_t h, uint32_t c) {
 // Column tiles per workgroup of the LDS-staged 128-row kernel (up to kMfmaLdsNkb
 // K-blocks) for a launch of `tiles` tiles: few column tiles make enough
 // workgroups of a small launch, many save a large one the start of each. us at
-// 8 / 16 / 32, launches of each in turn (NS = 1024; 512; 333, whose columns are
-// loaded by dwords):
+// 8 / 16 / 32, launches of each in turn, inputs and outputs changing from 800
+// tiles on (NS = 1024; 512; 333, whose columns are loaded by dwords):
 //   2 K-blocks     61 tiles 15.7 / 20.2 / 34.3; 15.7 / 22.8 / 38.1; 17.2 / 24.1 / 41.7
 //                 121: 29.4 / 26.6 / 38.0; 30.0 / 27.4 / 39.2; 29.9 / 30.4 / 42.5
 //               1,950: 483 / 486 / 500; 417 / 400 / 397; 408 / 404 / 407
 //   3              60: 17.6 / 25.8 / 43.3; 18.4 / 28.2 / 47.6; 21.1 / 30.7 / 53.8
 //                 239: 61.0 / 61.4 / 67.5; 62.4 / 63.0 / 69.1; 66.0 / 66.7 / 75.1
-//                 953: 250 / 228 / 253; 245 / 241 / 249; 254 / 251 / 264
-//               1,780: 495 / 470 / 467; 519 / 492 / 452; 475 / 465 / 460
+//                 846: 244 / 233 / 250; 256 / 245 / 241; 216 / 216 / 223
+//               1,238: 356 / 341 / 346; 372 / 356 / 340; 384 / 373 / 372
+//               1,933: 562 / 540 / 539; 599 / 576 / 526; 514 / 508 / 511
 //   4             116: 37.1 / 40.8 / 50.9; 39.5 / 41.4 / 54.8; 43.4 / 44.6 / 59.0
 //                 126: 44.5 / 42.0 / 52.2; 45.1 / 42.5 / 57.9; 50.0 / 46.3 / 59.6
 //                 141: 48.4 / 48.9 / 64.8; 48.4 / 51.9 / 66.2; 52.2 / 56.9 / 75.2
 //                 182: 58.5 / 56.3 / 69.5; 61.2 / 58.0 / 72.0; 66.8 / 64.8 / 78.6
-//                 948: 281 / 270 / 287; 276 / 273 / 284; 307 / 300 / 311
-//               1,152: 384 / 374 / 361; 328 / 324 / 320; 370 / 364 / 358
-//   5             999: 394 / 380 / 385; 369 / 366 / 369; 397 / 392 / 395
-//               1,098: 430 / 414 / 402; 395 / 394 / 389; 426 / 425 / 421
-//   6             928: 399 / 390 / 399; 389 / 389 / 393; 417 / 419 / 427
+//                 916: 296 / 280 / 284; 298 / 288 / 286; 307 / 290 / 310
+//               1,103: 357 / 340 / 329; 354 / 343 / 334; 377 / 370 / 364
+//   5             920: 349 / 337 / 340; 351 / 345 / 348; 365 / 365 / 373
+//                 980: 373 / 361 / 357; 372 / 367 / 361; 391 / 390 / 388
+//   6             899: 381 / 363 / 364; 377 / 369 / 381; 402 / 398 / 409
+//                 978: 413 / 400 / 391; 410 / 405 / 406; 439 / 437 / 434
 //               1,907: 819 / 794 / 777; 849 / 821 / 814; 915 / 885 / 873
 // Four K-blocks change over twice: 16 column tiles make 4 workgroups a tile, so
 // 128 tiles fill 256 CUs with two each and 192 with three, and 8 column tiles
 // split more evenly just past either (up to 120 tiles their 8 a tile and the
-// variance blocks all fit the chip at once).
+// variance blocks all fit the chip at once). From 900 tiles on 16 and 32 lie
+// within a few per cent of each other, either way by layout, until 32 wins.
 constexpr int kMfmaLdsNkb = 6;
 constexpr int wide_ntw(int nkb, uint32_t tiles) {
   const bool few = nkb <= 2   ? tiles < 100
@@ -62,8 +65,7 @@ constexpr int wide_ntw(int nkb, uint32_t tiles) {
                               : tiles <= 120 || (tiles > 128 && tiles <= 152) ||
                                     (tiles > 192 && tiles < 200);
   if (few) return 8;
-  const uint32_t many = nkb == 3 ? 1500 : nkb == 6 ? 950 : 1050;
-  return nkb > 2 && tiles >= many ? 32 : 16;
+  return nkb > 2 && tiles >= 900 ? 32 : 16;
 }
 
 // Column tiles of a batch's 128-row family of `tiles` tiles, whose bands run up
