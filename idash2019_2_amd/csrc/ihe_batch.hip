@@ -18,7 +18,11 @@
 // input words in LDS at three workgroups per CU, where the one kernel's
 // register budget (its largest body's) holds two workgroups per CU and its
 // 128-row bodies stage in registers; IHE_BATCH_PERSISTENT=1 asks for the one
-// kernel whenever it has a body for every family.
+// kernel whenever it has a body for every family. A batch of one-K-block families
+// alone keeps the one launch as its default, though one launch per family, which
+// takes the 16-byte kernel and needs no resident workgroups, is faster (n = 5,
+// unrotated: 2 cohorts of 300 targets 54.5 and 6.8 us, 16 of 2,000 184 and 135 us, 16
+// of 10,000 982 and 799 us); IHE_BATCH_PERSISTENT=0 asks for that.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -37,7 +41,7 @@ struct ihe_batch {
     bool rot;
     uint32_t entry0, num_entries, first0, num_items;
     uint32_t item0;  // first tile in the tile -> entry table
-    bool runs4;      // rotated 128-row family whose region sizes are multiples of 4
+    bool runs4;      // rotated 64- or 128-row family whose region sizes are multiples of 4
   };
   std::vector<Launch> launches;
   bool persistent = false;
@@ -70,7 +74,8 @@ struct Keyed {
   MfmaEntry e;
   uint32_t tiles, band_tiles;
   // rotated 128-row or one-K-block 64-row tiles whose region size is a multiple
-  // of 4: their own family, launched with 16-byte loads
+  // of 4: their own family, launched with 16-byte loads (in the one kernel, whose
+  // bodies load dwords, only a family more)
   bool runs4;
 };
 

@@ -41,7 +41,10 @@ struct alignas(16) MfmaEntry {
   uint32_t ns, rs, R, ct_base;  // layout; ct_base = first ciphertext of `in`
   uint32_t tile_base;           // first tile of the segment
   uint32_t pad0;
-  uint64_t rmagic;  // c / R = umul64hi(c, rmagic) for every 32-bit c (R > 1)
+  // ceil(2^64 / R) (R > 1): c / R = umul64hi(c, rmagic) for every 32-bit c and
+  // R <= 2^31 (the error c * (rmagic - 2^64 / R) / 2^64 stays below 2^-32, under
+  // the 1 / R gap of a non-integral quotient to the next integer)
+  uint64_t rmagic;
   uint32_t pad[10];
 };
 static_assert(sizeof(MfmaEntry) == 128, "entry is two 64-byte scalar loads");
@@ -79,17 +82,15 @@ struct VarEntry {
   const double *var_in;
   double *var_out;
   uint32_t num_out, R;
-  uint64_t rmagic;          // floor(2^64 / R), rounded up: div_r divides by its high word (R > 1)
+  uint32_t recip;           // floor(2^32 / R) (R > 1): the kernel's estimate of c / R
 };
 
-// The variance entry of one cohort: rmagic = floor((2^64 - 1) / R) + 1 makes
-// the high half of c * rmagic equal floor(c / R) for every 32-bit c and
-// 1 < R <= 2^31 (the error c * (rmagic - 2^64 / R) / 2^64 stays below 2^-32,
-// under the 1 / R gap of a non-integral quotient to the next integer).
+// The variance entry of one cohort.
 inline VarEntry make_var_entry(const uint32_t *blk_off, const uint32_t *col, const int32_t *w2,
                                const uint32_t *base, const double *var_in, double *var_out,
                                uint32_t num_out, uint32_t R) {
-  return {blk_off, col, w2, base, var_in, var_out, num_out, R, R > 1 ? UINT64_MAX / R + 1 : 0};
+  return {blk_off, col,     w2, base,
+          var_in,  var_out, num_out, R, R > 1 ? (uint32_t)((1ull << 32) / R) : 0};
 }
 // A packed entry's offset field for padding.
 constexpr uint32_t kVarPackedPad = 0xFFFFu;

@@ -348,7 +348,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_cloud_mfma1(MfmaArgs A) {
 // How it runs (launch_k1 chooses): kFew leaves the output to the infinity cache
 // (sc1 without nt) and keeps four sums per product, independent MFMAs at two
 // waves per SIMD; kFour the same with streaming stores; kTwo two sums at a time
-// (one shift's products into the higher sum, then the next), 158 registers and
+// (one shift's products into the higher sum, then the next), 159 registers and
 // three waves per SIMD, with the weights read from LDS and the results as whole
 // tuples until their stores. Rotated launches measured slower as kTwo (512
 // against 460 us).
@@ -756,10 +756,11 @@ void k_cloud_mfmaw(MfmaArgs A) {
 }
 
 // ---------------------------------------------------------------------------
-// 128-row tiles at three workgroups per CU. The product is k_cloud_mfmaw's;
-// the input words reach LDS by LDS-direct buffer loads (no load registers) and
-// the column words stay in LDS, so that a wave fits the 168 registers of three
-// waves per SIMD. A rotated column loads its words from their rotated places,
+// 128-row tiles at three workgroups per CU, four at 2 and 3 K-blocks and at 4 with
+// 16-byte staging loads. The product is k_cloud_mfmaw's; the input words reach LDS
+// by LDS-direct buffer loads (no load registers) and the column words stay in
+// LDS, so that a wave fits the 168 (128) registers of three (four) waves per
+// SIMD. A rotated column loads its words from their rotated places,
 // and the recoding negates those that wrapped past N. Per column tile: the
 // workgroup recodes the staged words into the B planes (one buffer), then
 // issues the next column tile's loads straight into the staging buffer and
@@ -1046,14 +1047,14 @@ void k_cloud_batch(PersistArgs P) {
 // ---------------------------------------------------------------------------
 // Output variances, 256 outputs per block.
 constexpr uint32_t kVarAhead = 8;
-// c / R for any 32-bit c: the estimate by floor(2^32 / R) (rmagic's high word) is
-// the quotient or one less.
-__device__ __forceinline__ uint32_t div_r(uint32_t c, uint32_t R, uint64_t rmagic, bool &whole) {
+// c / R for any 32-bit c: the estimate by recip = floor(2^32 / R) is the quotient
+// or one less.
+__device__ __forceinline__ uint32_t div_r(uint32_t c, uint32_t R, uint32_t recip, bool &whole) {
   if (R == 1) {
     whole = true;
     return c;
   }
-  const uint32_t q = __umulhi(c, (uint32_t)(rmagic >> 32)), rest = c - q * R;
+  const uint32_t q = __umulhi(c, recip), rest = c - q * R;
   whole = rest == 0 || rest == R;
   return q + (rest >= R ? 1 : 0);
 }
@@ -1113,7 +1114,7 @@ __device__ __forceinline__ void var_block(const VarArgs &A, uint32_t chunk, uint
         w2[j] = (int32_t)(aw * aw);
       }
       bool whole;
-      const uint32_t ct = div_r(cj, E.R, E.rmagic, whole);
+      const uint32_t ct = div_r(cj, E.R, E.recip, whole);
       keep[j] = !pad && whole && e + j < e1;
       x[j] = E.var_in[keep[j] ? ct : 0];
     }

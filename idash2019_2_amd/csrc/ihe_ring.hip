@@ -200,8 +200,8 @@ __device__ __forceinline__ void noise_sample4(const uint64_t u[4], const uint64_
 // so decryption is the product of the ciphertexts' a-rows with one Toeplitz
 // matrix of entries in {-1, 0, 1}. Each a word is recoded into balanced
 // signed bytes (x = sum_p 2^(8p) d_p, d_p = byte_p(x + 0x80808080) - 128), one
-// v_mfma_i32_32x32x32_i8 per byte plane and K-block of 32 coefficients, four
-// int32 accumulators recombined with shifts mod 2^32 (|partial| <= 2^17).
+// v_mfma_i32_32x32x32_i8 per byte plane and K-block of 32 coefficients, all into
+// one int32 accumulator that wraps mod 2^32.
 //
 // Work items are 32 ciphertexts x 8 TPW column tiles of 32 words (TPW = 1 .. 4
 // tiles a wave; all 1,024 words at TPW = 4). One workgroup of 8 waves per CU
