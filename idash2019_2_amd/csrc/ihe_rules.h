@@ -32,8 +32,8 @@ constexpr uint32_t ring_run(uint32_t nt, uint32_t h, uint32_t c) {
 // Column tiles per workgroup of the LDS-staged 128-row kernel (up to kMfmaLdsNkb
 // K-blocks) for a launch of `tiles` tiles: few column tiles make enough
 // workgroups of a small launch, many save a large one the start of each. us at
-// 8 / 16 / 32, launches of each in turn, inputs and outputs changing from 800
-// tiles on (NS = 1024; 512; 333, whose columns are loaded by dwords):
+// 8 / 16 / 32, launches of each in turn, at 800 to 1,300 tiles with changing
+// inputs and outputs (NS = 1024; 512; 333, whose columns are loaded by dwords):
 //   2 K-blocks     61 tiles 15.7 / 20.2 / 34.3; 15.7 / 22.8 / 38.1; 17.2 / 24.1 / 41.7
 //                 121: 29.4 / 26.6 / 38.0; 30.0 / 27.4 / 39.2; 29.9 / 30.4 / 42.5
 //               1,950: 483 / 486 / 500; 417 / 400 / 397; 408 / 404 / 407

@@ -166,7 +166,7 @@ int ihe_band_create(ihe_ctx *ctx, const ihe_layout *layout, uint32_t num_in_cts,
 /* Autotuner: compiles the model once per feasible MFMA tile shape (output rows
  * per tile, i.e. targets per workgroup; K-blocks of 32 columns, the window
  * length a tile covers; 32-word column tiles per wave, the coefficient chunk),
- * times `reps` cloud launches of each on the caller's cohort buffers (d_out is
+ * times at least `reps` cloud launches of each on the caller's cohort buffers (d_out is
  * overwritten) and returns the fastest band in *out. results[0 .. *num_results)
  * receive the timings (*num_results: capacity in, count out). Needs weights
  * within the MFMA split; IHE_ERR_UNSUPPORTED otherwise. */
